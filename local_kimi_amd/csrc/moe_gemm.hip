@@ -316,7 +316,13 @@ schedule_one_kernel(const RouteTable rt, int64_t n, Schedule sc, const float* __
 
 // weight format x activation type; kFmtMxF8: MXFP4 weights x activations
 // split into fp8 hi + lo with per-32 E8M0 exponents (scaled fp4 MFMA)
-enum : int { kFmtW4A16 = 0, kFmtMxBf16 = 1, kFmtMxF16 = 2, kFmtMxF8 = 3 };
+// kFmtW4G32 / kFmtW4G64: W4A16 with groups of 32 / 64 on 16-byte weight loads
+// (transpose4), in kernels whose kFmtW4A16 form takes G = 128 only
+enum : int { kFmtW4A16 = 0, kFmtMxBf16 = 1, kFmtMxF16 = 2, kFmtMxF8 = 3, kFmtW4G32 = 4, kFmtW4G64 = 5 };
+constexpr bool fmt_is_w4(int fmt) { return fmt == kFmtW4A16 || fmt == kFmtW4G32 || fmt == kFmtW4G64; }
+// group width of the 16-byte-load W4A16 forms, and their MFMAs (32 of k) per group
+constexpr int fmt_group(int fmt) { return fmt == kFmtW4G32 ? 32 : fmt == kFmtW4G64 ? 64 : 128; }
+constexpr int fmt_chain(int fmt) { return fmt_group(fmt) / 32; }
 enum : int { kActSwiglu = 0, kActSitu = 1 };                   // two-matrix epilogues
 
 struct GemmArgs {
@@ -395,6 +401,31 @@ __device__ inline bf16x8_t unpack_q8(uint32_t w) {
   const u32x4_t v = {(w & kPairMask) ^ kFlip128, ((w >> 4) & kPairMask) ^ kFlip128,
                      ((w >> 8) & kPairMask) ^ kFlip128, ((w >> 12) & kPairMask) ^ kFlip128};
   return __builtin_bit_cast(bf16x8_t, v);
+}
+
+// W4A16 groups narrower than a k-step on 16-byte loads: lane block jq = lane / 16
+// loads codes 32 jq .. 32 jq + 31 of its column, but an MFMA must stay inside
+// one group, so MFMA t takes codes 32 t .. 32 t + 31 and lane block jq needs
+// dword jq of block t: a 4 x 4 transpose over (dword, lane block), two
+// half-wave swaps and two row swaps. The four dwords loaded apart (and four
+// 2-byte scales) are eight loads a k-step instead of two: at 16 tokens of the
+// Kimi-Linear layer with G = 32 they held the block to 1.0 TB/s, 416 us with
+// its norms and router, against 147 us on the persistent kernel in this form.
+__device__ inline void transpose4(uint32_t (&w)[4]) {
+  auto half = [](uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+  };
+  auto row = [](uint32_t& a, uint32_t& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = r[0];
+    b = r[1];
+  };
+  half(w[0], w[2]);
+  half(w[1], w[3]);
+  row(w[0], w[1]);
+  row(w[2], w[3]);
 }
 
 // 2**(e - 127) as fp32 for an E8M0 byte (e = 0: the subnormal 2**-127, 255: inf)
@@ -1693,17 +1724,26 @@ constexpr int kPsEarlyPairs = 1;  // ring pairs issued before the first staging 
 template <int FMT>
 __device__ inline void ps_stage_store(uint4* afrag, float* offs, int frag, int c, int mr,
                                       const uint4 v) {
-  const int t = c & 3, j = c >> 2;  // 16-byte unit c of the step feeds MFMA t, lane block j
+  // 16-byte unit c of the step feeds MFMA t, lane block j (groups of 32 and 64:
+  // the MFMAs take k in order, see transpose4)
+  constexpr int kChain = fmt_chain(FMT);
+  const int t = kChain < 4 ? c >> 2 : c & 3, j = kChain < 4 ? c & 3 : c >> 2;
   uint4* dst = &afrag[(frag + t) * kWave + j * 16 + (mr ^ (4 * t + j))];
-  if constexpr (FMT != kFmtW4A16) {
+  if constexpr (!fmt_is_w4(FMT)) {
     *dst = v;
   } else {
     uint32_t q[4];
     pair_x8(v, q);
     *dst = make_uint4(q[0], q[1], q[2], q[3]);
-    float sx = sum8(sum_x8_dot(v));
-    sx += dpp_f32<kRowMirror>(sx);  // the 16 units of a (row, step) sit in one 16-lane row
-    if (c == 0) offs[frag * 16 + mr] = -kCodeOffset * sx;
+    float sx = sum_x8_dot(v);  // the 16 units of a (row, step) sit in one 16-lane row
+    if constexpr (kChain == 4) {
+      sx = sum8(sx);
+      sx += dpp_f32<kRowMirror>(sx);
+    } else {
+      sx = sum4(sx);
+      if constexpr (kChain == 2) sx += dpp_f32<kRowHalfMirror>(sx);
+    }
+    if ((c & (4 * kChain - 1)) == 0) offs[(frag + t / kChain) * 16 + mr] = -kCodeOffset * sx;
   }
 }
 
@@ -1712,13 +1752,13 @@ __device__ inline void ps_stage_store(uint4* afrag, float* offs, int frag, int c
 // are issued back to back (they are the two halves of one 128-byte line of
 // the weight row, so the line is fetched once: requested apart, each half
 // costs a fetch of its own), and one scale load serves both steps (W4A16
-// G = 128: the bf16 pair, low half = step 2q; MXFP4: eight E8M0 bytes, four
-// per step). Whole-dword scale loads keep the ring free of narrow loads, whose
+// G = 128: the bf16 pair, low half = step 2q; G = 64 and 32: four and eight
+// bf16; MXFP4: eight E8M0 bytes, four per step). Whole-dword scale loads keep the ring free of narrow loads, whose
 // zero-extension the compiler otherwise places at the loop latch, where it
 // waits for every load in flight.
 template <int FMT, int MATS, int NT>
 struct PsPair {
-  static constexpr int kSw = FMT == kFmtW4A16 ? 1 : 2;  // scale dwords per pair
+  static constexpr int kSw = fmt_is_w4(FMT) ? 4 / fmt_chain(FMT) : 2;  // scale dwords per pair
   uint32_t w[2][MATS][NT][4];
   uint32_t s[MATS][NT][kSw];
 
@@ -1731,13 +1771,19 @@ struct PsPair {
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         const void* sp;
-        if constexpr (FMT == kFmtW4A16)
-          sp = static_cast<const uint16_t*>(srow[mi][nt]) + step0;
+        if constexpr (fmt_is_w4(FMT))
+          sp = static_cast<const uint16_t*>(srow[mi][nt]) + step0 * (4 / fmt_chain(FMT));
         else
           sp = static_cast<const uint8_t*>(srow[mi][nt]) + static_cast<int64_t>(step0) * 4;
         if (!live) sp = dummy;
         if constexpr (kSw == 1) {
           s[mi][nt][0] = *static_cast<const uint32_t*>(sp);
+        } else if constexpr (kSw == 4) {
+          const uint4 v = *static_cast<const uint4*>(sp);
+          s[mi][nt][0] = v.x;
+          s[mi][nt][1] = v.y;
+          s[mi][nt][2] = v.z;
+          s[mi][nt][3] = v.w;
         } else {
           const uint2 v = *static_cast<const uint2*>(sp);
           s[mi][nt][0] = v.x;
@@ -1954,7 +2000,7 @@ template <int FMT, int MATS, int DEPTH, bool GATHER, bool SCATTER, bool SPLIT = 
           bool SWI = false, bool ROUTED = false>
 __global__ void __launch_bounds__(kStWaves * kWave)
 w4a16_persist_kernel(const GemmArgs g, int nbuf) {
-  static_assert(FMT == kFmtW4A16 || FMT == kFmtMxBf16, "bf16 activations, 16-byte weight loads");
+  static_assert(fmt_is_w4(FMT) || FMT == kFmtMxBf16, "bf16 activations, 16-byte weight loads");
   static_assert(!ROUTED || (GATHER && !SWI), "routing feeds the gate/up GEMM");
   static_assert(DEPTH % 2 == 0, "the ring holds pairs of k-steps");
   static_assert(!SPLIT || MATS == 1, "split units hold one matrix");
@@ -1966,7 +2012,7 @@ w4a16_persist_kernel(const GemmArgs g, int nbuf) {
   // 43.1 us with 32-column units, whose longer last units stretch the tail
   constexpr int NT = 1;
   constexpr int kHalfCap = SWI ? kPsSwiHalfMax : kPsHalfMax;
-  constexpr bool kMx = FMT != kFmtW4A16;
+  constexpr bool kMx = !fmt_is_w4(FMT);
   extern __shared__ uint4 smem[];
   __shared__ int64_t seg_row[kPsMaxSegs][16];  // activation row of tile row m
   __shared__ int32_t seg_out[kPsMaxSegs][16];  // output row of tile row m
@@ -2256,6 +2302,45 @@ w4a16_persist_kernel(const GemmArgs g, int nbuf) {
             tot[mi][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                 af, __builtin_bit_cast(bf16x8_t, unpack_fp4x8_bf16(wj.w[h][mi][nt][t], sc[mi][nt])),
                 tot[mi][nt], 0, 0, 0);
+      }
+    } else if constexpr (fmt_chain(FMT) < 4) {
+      // groups of 32 or 64 inside the step: kChain MFMAs from the group's
+      // offset, closed by one FMA per output, in k order
+      constexpr int kChain = fmt_chain(FMT), kGroups4 = 4 / kChain;
+      float sc[MATS][NT][kGroups4];
+      uint32_t wt[MATS][NT][4];
+#pragma unroll
+      for (int mi = 0; mi < MATS; ++mi)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+#pragma unroll
+          for (int q = 0; q < kGroups4; ++q) {  // decoded as below
+            const int e = h * kGroups4 + q;
+            if (e & 1)
+              asm("v_and_b32 %0, 0xffff0000, %1" : "=v"(sc[mi][nt][q]) : "v"(wj.s[mi][nt][e >> 1]));
+            else
+              asm("v_lshlrev_b32 %0, 16, %1" : "=v"(sc[mi][nt][q]) : "v"(wj.s[mi][nt][e >> 1]));
+          }
+#pragma unroll
+          for (int t = 0; t < 4; ++t) wt[mi][nt][t] = wj.w[h][mi][nt][t];
+          transpose4(wt[mi][nt]);
+        }
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const bf16x8_t af = __builtin_bit_cast(
+            bf16x8_t, afrag[(frag0 + t) * kWave + jq * 16 + (ln ^ (4 * t + jq))]);
+        const bool first = t % kChain == 0, last = (t + 1) % kChain == 0;
+        f32x4_t neg = zero4;
+        if (first)
+          neg = *reinterpret_cast<const f32x4_t*>(&offs[(frag0 + t / kChain) * 16 + jq * 4]);
+#pragma unroll
+        for (int mi = 0; mi < MATS; ++mi)
+#pragma unroll
+          for (int nt = 0; nt < NT; ++nt) {
+            acc[mi][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                af, unpack_q8(wt[mi][nt][t]), first ? neg : acc[mi][nt], 0, 0, 0);
+            if (last) tot[mi][nt] += sc[mi][nt][t / kChain] * acc[mi][nt];
+          }
       }
     } else {
       // the bf16 scale is decoded first, by an instruction the register
@@ -2906,13 +2991,22 @@ constexpr int kPsNotApplicable = -1000;
 template <int FMT, int MATS>
 int persist_launch(const GemmArgs& g, Mode mode, int64_t tiles_bound, hipStream_t s,
                    const char* what, PsForm form = PsForm::Plain, bool launch = true) {
-  if constexpr (FMT != kFmtW4A16 && FMT != kFmtMxBf16) {
+  if constexpr (!fmt_is_w4(FMT) && FMT != kFmtMxBf16) {
     return kPsNotApplicable;
   } else {
     if (persist_disabled() || mode == Mode::Dense || g.outputs != 1) return kPsNotApplicable;
-    // W4A16: G = 128 and an even number of groups per row (dword scale pairs stay in the row)
-    if (g.k % 128 != 0 || (FMT == kFmtW4A16 && (g.group != 128 || g.k % 256 != 0)))
+    // W4A16: the form's group, and an even number of k-steps per row (the scales
+    // of a pair of steps are one load, aligned in every row)
+    if (g.k % 128 != 0 || (fmt_is_w4(FMT) && (g.group != fmt_group(FMT) || g.k % 256 != 0)))
       return kPsNotApplicable;
+    // groups of 32 and 64 were taken at any alignment of the banks (4-byte
+    // weight and 2-byte scale loads), so others keep the per-tile kernel
+    if (fmt_is_w4(FMT) && FMT != kFmtW4A16) {
+      uintptr_t any = 0;
+      for (int mi = 0; mi < 2; ++mi)
+        any |= reinterpret_cast<uintptr_t>(g.wp[mi]) | reinterpret_cast<uintptr_t>(g.ws[mi]);
+      if (any & 15) return kPsNotApplicable;
+    }
     const size_t one = stream_lds_bytes(g.k, 1);
     const int nbuf = 2 * one <= static_cast<size_t>(kPsMaxLds) ? 2 : (one <= static_cast<size_t>(kPsMaxLds) ? 1 : 0);
     if (nbuf == 0) return kPsNotApplicable;
@@ -2971,6 +3065,19 @@ int persist_launch(const GemmArgs& g, Mode mode, int64_t tiles_bound, hipStream_
   }
 }
 
+// The same for the weight format's group width (W4A16: 128, 64 or 32).
+template <int FMT, int MATS>
+int persist_format(const GemmArgs& g, Mode mode, int64_t tiles_bound, hipStream_t s,
+                   const char* what, PsForm form = PsForm::Plain, bool launch = true) {
+  if constexpr (FMT == kFmtW4A16) {
+    if (g.group == 32)
+      return persist_launch<kFmtW4G32, MATS>(g, mode, tiles_bound, s, what, form, launch);
+    if (g.group == 64)
+      return persist_launch<kFmtW4G64, MATS>(g, mode, tiles_bound, s, what, form, launch);
+  }
+  return persist_launch<FMT, MATS>(g, mode, tiles_bound, s, what, form, launch);
+}
+
 template <int FMT, int MATS>
 int stream_launch(GemmArgs g, Mode mode, int64_t tiles, int mt, hipStream_t s, const char* what) {
   constexpr int NT = MATS == 2 ? 1 : 2;
@@ -3010,8 +3117,8 @@ int stream_launch(GemmArgs g, Mode mode, int64_t tiles, int mt, hipStream_t s, c
     if (mt == 1) stream_dispatch<FMT, MATS, 1, true>(g, mode, nb, lds, s);
     else stream_dispatch<FMT, MATS, 4, true>(g, mode, nb, lds, s);
   } else if (mt == 1) {
-    if (wide) {
-      const int rc = persist_launch<FMT, MATS>(g, mode, tiles, s, what);
+    if (wide || FMT == kFmtW4A16) {
+      const int rc = persist_format<FMT, MATS>(g, mode, tiles, s, what);
       if (rc != kPsNotApplicable) return rc;
     }
     if (wide) stream_dispatch<FMT, MATS, 1, kWideOk>(g, mode, nb, lds, s);
@@ -3101,8 +3208,8 @@ int moe_act_mult(int64_t entries) { return stream_tile_mt(entries) == 1 ? 2 : 1;
 template <int MATS>
 int persist_fmt(bool mx, const GemmArgs& g, Mode mode, int64_t tiles_bound, hipStream_t s,
                 const char* what, PsForm form, bool launch) {
-  if (mx) return persist_launch<kFmtMxBf16, MATS>(g, mode, tiles_bound, s, what, form, launch);
-  return persist_launch<kFmtW4A16, MATS>(g, mode, tiles_bound, s, what, form, launch);
+  if (mx) return persist_format<kFmtMxBf16, MATS>(g, mode, tiles_bound, s, what, form, launch);
+  return persist_format<kFmtW4A16, MATS>(g, mode, tiles_bound, s, what, form, launch);
 }
 
 // W4A16: a power-of-two group (multiple of 32) dividing k; MXFP4: 32.

@@ -257,3 +257,39 @@ def test_split_swiglu_matches_the_fused_epilogue(rng, weights, tokens):
         eo = X.grouped(act.reshape(len(sel) * (k + 1), -1), stable.reshape(-1, 1), sub[4], sub[5])
         ey = OM.combine(eo.reshape(len(sel), k + 1, -1), cw)
     assert_close_bf16(to_bits(y)[sel], ey, what=f"{weights} split SwiGLU T={tokens}")
+
+
+@pytest.mark.parametrize("group", [32, 64])
+@pytest.mark.parametrize("h,inter,tokens", [(768, 512, 40), (512, 768, 13), (1024, 512, 3),
+                                            (1024, 768, 21)])
+def test_moe_block_narrow_groups_match_per_tile_and_oracle(rng, monkeypatch, group, h, inter,
+                                                           tokens):
+    """Groups of 32 and 64 on 16-byte loads (codes transposed between lane
+    blocks) against the per-tile kernel's 4-byte loads: the same MFMA chains
+    and group sums, so the same bits; every ring depth."""
+    from local_kimi_amd.kernels import w4a16_moe_forward
+
+    e_routed, k = 24, 4
+    banks = (*_w4_bank(rng, e_routed + 1, inter, h, group),
+             *_w4_bank(rng, e_routed + 1, inter, h, group),
+             *_w4_bank(rng, e_routed + 1, h, inter, group))
+    x = random_bf16_bits(rng, (tokens, h))
+    logits = rng.normal(0, 1, (tokens, e_routed)).astype(np.float32)
+    dev_banks = [_dev(b) for b in banks]
+    args = (_dev(x), _dev(logits), None, *dev_banks, k, 2.446)
+    (y, idx, _), (y0, idx0, _) = _both(monkeypatch, w4a16_moe_forward, *args)
+    assert torch.equal(idx, idx0)
+    assert torch.equal(y, y0), "persistent and per-tile kernels differ"
+    ey, eidx, _ = OM.moe_block(x, logits, None, *banks, top_k=k, routed_scaling_factor=2.446,
+                               group_size=group)
+    assert np.array_equal(idx.cpu().numpy(), eidx)
+    assert_close_bf16(to_bits(y), ey, what=f"G={group} moe block h={h} i={inter} T={tokens}")
+
+    # banks at a 4-byte offset, which the per-tile kernel has always taken
+    def shifted(t):
+        buf = torch.empty(t.numel() * t.element_size() + 4, dtype=torch.uint8, device=DEV)
+        out = buf[4:].view(t.dtype).view(t.shape)
+        return out.copy_(t)
+
+    moved = (args[0], args[1], None, *(shifted(b) for b in dev_banks), k, 2.446)
+    assert torch.equal(w4a16_moe_forward(*moved)[0], y)
