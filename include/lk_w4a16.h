@@ -72,6 +72,12 @@ LK_API int lk_get_path(const char* knob);
 LK_API int lk_w4a16_quantise(const uint16_t* weight, uint8_t* packed, uint16_t* scales,
                       int64_t n, int64_t k, int64_t group_size, void* stream);
 
+/* lk_w4a16_quantise, and *nonfinite (device memory, zeroed by the caller; null:
+ * not wanted) becomes 1 if any weight is infinite or NaN. */
+LK_API int lk_w4a16_quantise_checked(const uint16_t* weight, uint8_t* packed, uint16_t* scales,
+                                     int32_t* nonfinite, int64_t n, int64_t k,
+                                     int64_t group_size, void* stream);
+
 /* packed + scales -> out [N,K]: bf16(q * scale) as bf16 when out_f32 == 0,
  * or the exact q * scale as float32 when out_f32 != 0. */
 LK_API int lk_w4a16_dequantise(const uint8_t* packed, const uint16_t* scales, void* out,

@@ -24,6 +24,7 @@ _I = ctypes.c_int
 # name -> argument types (every entry point returns int status)
 SIGNATURES: dict[str, list] = {
     "lk_w4a16_quantise": [_P, _P, _P, _I64, _I64, _I64, _P],
+    "lk_w4a16_quantise_checked": [_P, _P, _P, _P, _I64, _I64, _I64, _P],
     "lk_w4a16_dequantise": [_P, _P, _P, _I64, _I64, _I64, _I, _P],
     "lk_w4a16_dense": [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _P],
     "lk_w4a16_dense_reference": [_P, _P, _P, _P, _I64, _I64, _I64, _I64, _P],

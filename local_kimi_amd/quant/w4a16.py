@@ -77,15 +77,17 @@ def quantise(weight: torch.Tensor, *, group_size: int = GROUP_SIZE) -> W4A16Tens
     _check_group(weight.shape[1], group_size)
     if weight.device.type != "cuda":
         raise ValueError("the HIP W4A16 quantiser requires a CUDA (HIP) tensor")
-    if not bool(torch.isfinite(weight).all()):
-        raise ValueError("weight must contain only finite values")
     n, k = weight.shape
     w = weight.detach().contiguous()
     packed = torch.empty((n, k // 2), dtype=torch.uint8, device=weight.device)
     scales = torch.empty((n, k // group_size), dtype=SCALE_DTYPE, device=weight.device)
+    nonfinite = torch.zeros((1,), dtype=torch.int32, device=weight.device)
     with torch.cuda.device(weight.device):
-        _lib.call("lk_w4a16_quantise", w.data_ptr(), packed.data_ptr(), scales.data_ptr(), n, k,
-                  group_size, torch.cuda.current_stream(weight.device).cuda_stream)
+        _lib.call("lk_w4a16_quantise_checked", w.data_ptr(), packed.data_ptr(), scales.data_ptr(),
+                  nonfinite.data_ptr(), n, k, group_size,
+                  torch.cuda.current_stream(weight.device).cuda_stream)
+    if nonfinite.item():
+        raise ValueError("weight must contain only finite values")
     return W4A16Tensor(packed=packed, scales=scales, original_shape=(n, k), group_size=group_size)
 
 

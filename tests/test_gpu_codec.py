@@ -1,0 +1,66 @@
+"""The W4A16 quantiser's wide kernel (groups of 32, 64, 128) against the oracle,
+bit for bit: exact ties, zero groups, subnormal, tiny and huge groups (whose
+quotients leave the corrected-reciprocal range), group counts that do not fill
+a block, weights at an address that takes the one-thread-per-group kernel, and
+the non-finite check."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import w4a16 as OW
+from oracle.bf16 import f32_to_bf16_bits
+
+from ._helpers import from_bits, to_bits
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _require_gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("needs a GPU")
+
+
+def _weights(rng, n, k):
+    w = rng.normal(0, 0.02, (n, k)).astype(np.float32)
+    w[0, :] = 0.0
+    w[1 % n, :] = 1e-39                                    # subnormal
+    w[2 % n, :] = rng.normal(0, 1, k) * np.float32(2.0**-120)
+    w[3 % n, :] = rng.normal(0, 1, k) * np.float32(2.0**100)
+    w[4 % n, :] = (np.arange(k) % 29 - 14) * 0.5           # absmax 7: every half is a tie
+    w[5 % n, :] = ((np.arange(k) % 29 - 14) * 0.5) * 2.0**-95
+    return f32_to_bf16_bits(w)
+
+
+@pytest.mark.parametrize("group", [32, 64, 128, 256])
+@pytest.mark.parametrize("n,k", [(7, 256), (33, 768)])
+@pytest.mark.parametrize("shift", [0, 2])
+def test_quantise_matches_oracle(rng, group, n, k, shift):
+    from local_kimi_amd.quant import quantise
+
+    bits = _weights(rng, n, k)
+    flat = torch.empty(n * k + 8, dtype=torch.bfloat16, device=DEV)
+    w = flat[shift:shift + n * k].view(n, k)  # shift 2: a 4-byte aligned address
+    w.copy_(from_bits(bits, DEV))
+    got = quantise(w, group_size=group)
+    packed, scales = OW.quantise(bits, group)
+    assert np.array_equal(to_bits(got.scales), scales)
+    assert np.array_equal(got.packed.cpu().numpy(), packed)
+
+
+@pytest.mark.parametrize("group", [32, 64, 128, 256])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+def test_quantise_rejects_non_finite(rng, group, bad):
+    from local_kimi_amd.quant import quantise
+
+    w = torch.randn(5, 512, device=DEV).to(torch.bfloat16)
+    w[4, 511] = bad
+    with pytest.raises(ValueError, match="finite"):
+        quantise(w, group_size=group)
+    w[4, 511] = 0.0
+    quantise(w, group_size=group)
