@@ -17,6 +17,8 @@
 
 #include <stdlib.h>
 
+#include <algorithm>
+
 #include "lk_common.hpp"
 #include "lk_route.hpp"
 
@@ -1059,9 +1061,15 @@ constexpr size_t kMaxLds = 64 * 1024;
 // in lane order). Every output therefore has the same summation order whatever
 // the batch size, so a token's logits (and its routing) do not depend on the
 // batch, and reruns are bit-identical.
+// From kLogitWideTokens tokens router_logits_wide_kernel does the same sums
+// for kLogitExperts experts per wave: the loop above is bound by the VALU, a
+// third of it the multiply-adds and the rest the widening of x and w and the
+// reduction; with the weights widened once per wave, x once per token for all
+// of the wave's experts and the group sums added by one lane per output
+// (through LDS), 777 tokens x 256 experts x 2304 take 26 us instead of 68.
 constexpr int kLogitWaves = 4;
 constexpr int kLogitIters = 8;   // chunks per lane: h <= 64 * 8 * 8 = 4096
-constexpr int kLogitTokens = 16;  // tokens per wave (the weight row is reused)
+constexpr int kLogitTokens = 16;  // most tokens per wave (the weight row is reused)
 
 // WORDS = 16-byte loads per 8-value weight chunk: 1 (bf16) or 2 (fp32)
 template <int WORDS>
@@ -1109,14 +1117,15 @@ __device__ inline float logit_dot(const uint4 (&xv)[kLogitIters], const LogitRow
 template <int WORDS>
 __global__ void __launch_bounds__(kLogitWaves * 64)
 router_logits_kernel(const uint16_t* __restrict__ x, const void* __restrict__ w,
-                     float* __restrict__ logits, int64_t tokens, int64_t experts, int64_t h) {
+                     float* __restrict__ logits, int64_t tokens, int64_t experts, int64_t h,
+                     int tile) {
   const int wave = static_cast<int>(threadIdx.x) / kWave;
   const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
   const int64_t e = static_cast<int64_t>(blockIdx.x) * kLogitWaves + wave;
-  const int64_t t0 = static_cast<int64_t>(blockIdx.y) * kLogitTokens;
+  const int64_t t0 = static_cast<int64_t>(blockIdx.y) * tile;
   if (e >= experts) return;  // wave-uniform
   const int64_t chunks = h / 8;
-  const int nt = static_cast<int>(min<int64_t>(kLogitTokens, tokens - t0));
+  const int nt = static_cast<int>(min<int64_t>(tile, tokens - t0));
   const uint4* wrow = reinterpret_cast<const uint4*>(w) + e * chunks * WORDS;
   LogitRow<WORDS> wv;
   uint4 xv[kLogitIters];
@@ -1143,6 +1152,98 @@ router_logits_kernel(const uint16_t* __restrict__ x, const void* __restrict__ w,
   }
 }
 
+constexpr int kLogitExperts = 4;      // experts per wave (fewer where rows are wide)
+constexpr int64_t kLogitWideTokens = 64;
+constexpr int kLogitWideTile = 32;    // most tokens per wave
+
+// ITERS = chunks per lane, NE = experts per wave: ITERS * NE * 8 weight registers
+template <int WORDS, int ITERS, int NE>
+__global__ void __launch_bounds__(kLogitWaves * 64)
+router_logits_wide_kernel(const uint16_t* __restrict__ x, const void* __restrict__ w,
+                          float* __restrict__ logits, int64_t tokens, int64_t experts, int64_t h,
+                          int tile) {
+  // group sums of the wave's outputs: [token][expert][8 groups of 8 lanes]
+  __shared__ float part[kLogitWaves][kLogitWideTile * NE][9];
+  const int wave = static_cast<int>(threadIdx.x) / kWave;
+  const int lane = static_cast<int>(threadIdx.x) & (kWave - 1);
+  const int64_t e0 = (static_cast<int64_t>(blockIdx.x) * kLogitWaves + wave) * NE;
+  const int64_t t0 = static_cast<int64_t>(blockIdx.y) * tile;
+  if (e0 >= experts) return;  // wave-uniform, and no block barrier below
+  const int chunks = static_cast<int>(h / 8);
+  const int nt = static_cast<int>(min<int64_t>(tile, tokens - t0));
+  float wf[NE][ITERS][8];
+#pragma unroll
+  for (int n = 0; n < NE; ++n) {
+    const int64_t e = e0 + n < experts ? e0 + n : experts - 1;
+    const uint4* wrow = reinterpret_cast<const uint4*>(w) + e * chunks * WORDS;
+#pragma unroll
+    for (int i = 0; i < ITERS; ++i) {
+      const int c = lane + kWave * i;
+      const int cc = c < chunks ? c : 0;
+      uint32_t b[WORDS * 4];
+#pragma unroll
+      for (int q = 0; q < WORDS; ++q) {
+        const uint4 v = wrow[cc * WORDS + q];
+        b[4 * q] = v.x;
+        b[4 * q + 1] = v.y;
+        b[4 * q + 2] = v.z;
+        b[4 * q + 3] = v.w;
+      }
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        wf[n][i][j] = WORDS == 2 ? __uint_as_float(b[j])
+                                 : bf16_to_f32((j & 1) ? (b[j >> 1] >> 16) : (b[j >> 1] & 0xFFFFu));
+    }
+  }
+  const uint4* xr = reinterpret_cast<const uint4*>(x + t0 * h);
+  uint4 xv[ITERS];
+  auto load_x = [&](int t) {
+#pragma unroll
+    for (int i = 0; i < ITERS; ++i) {
+      const int c = lane + kWave * i;
+      xv[i] = xr[static_cast<int64_t>(t) * chunks + (c < chunks ? c : 0)];
+    }
+  };
+  load_x(0);
+  for (int t = 0; t < nt; ++t) {
+    float acc[NE];
+#pragma unroll
+    for (int n = 0; n < NE; ++n) acc[n] = 0.f;
+#pragma unroll
+    for (int i = 0; i < ITERS; ++i) {
+      const bool ok = lane + kWave * i < chunks;  // a chunk past the row keeps acc
+      const uint32_t a[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w};
+      float xf[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        xf[j] = bf16_to_f32((j & 1) ? (a[j >> 1] >> 16) : (a[j >> 1] & 0xFFFFu));
+#pragma unroll
+      for (int n = 0; n < NE; ++n) {
+        float p = acc[n];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) p = fmaf(xf[j], wf[n][i][j], p);
+        acc[n] = ok ? p : acc[n];
+      }
+    }
+    if (t + 1 < nt) load_x(t + 1);  // wave-uniform
+#pragma unroll
+    for (int n = 0; n < NE; ++n) {
+      const float g8 = sum8(acc[n]);
+      if ((lane & 7) == 0) part[wave][t * NE + n][lane >> 3] = g8;
+    }
+  }
+  // one lane per output: the 8 group sums in lane order (LDS operations of one
+  // wave complete in order)
+  __builtin_amdgcn_wave_barrier();
+  for (int o = lane; o < nt * NE; o += kWave) {
+    float total = 0.f;
+#pragma unroll
+    for (int gidx = 0; gidx < 8; ++gidx) total += part[wave][o][gidx];
+    const int64_t e = e0 + o % NE;
+    if (e < experts) logits[(t0 + o / NE) * experts + e] = total;
+  }
+}
+
 }  // namespace
 }  // namespace lk
 
@@ -1165,14 +1266,39 @@ int lk_router_logits(const uint16_t* x, const void* w, float* logits, int64_t to
              "too many tokens or experts for one call");
   if (tokens == 0) return LK_OK;
   LK_REQUIRE(x != nullptr, "null activation pointer");
+  if (tokens >= kLogitWideTokens) {
+    const bool narrow = h <= 64 * 8 * 5;
+    const int ne = narrow ? kLogitExperts : kLogitExperts / 2;
+    const int64_t cols = (experts + kLogitWaves * ne - 1) / (kLogitWaves * ne);
+    // tokens per wave: whole rounds of 512 blocks (two fit a CU)
+    const int64_t slots = 512 * ((tokens * cols + 512 * kLogitWideTile - 1) / (512 * kLogitWideTile));
+    const int64_t rows = std::max<int64_t>(1, slots / cols);  // token tiles
+    const int tile = static_cast<int>(
+        std::min<int64_t>(kLogitWideTile, std::max<int64_t>(4, (tokens + rows - 1) / rows)));
+    const int64_t tiles = (tokens + tile - 1) / tile;
+    if (tiles <= 65535) {
+      const dim3 wide(static_cast<unsigned>(cols), static_cast<unsigned>(tiles));
+      auto* fn = weight_f32 ? (narrow ? &router_logits_wide_kernel<2, 5, kLogitExperts>
+                                      : &router_logits_wide_kernel<2, 8, kLogitExperts / 2>)
+                            : (narrow ? &router_logits_wide_kernel<1, 5, kLogitExperts>
+                                      : &router_logits_wide_kernel<1, 8, kLogitExperts / 2>);
+      fn<<<wide, kLogitWaves * kWave, 0, as_stream(stream)>>>(x, w, logits, tokens, experts, h,
+                                                              tile);
+      return check_launch("lk_router_logits");
+    }
+  }
+  // tokens per wave (the weight row is reused): fewer where the waves are few
+  // (16 tokens x 256 experts: 2 a wave instead of 16, 4.6 us instead of 12.8)
+  int tile = kLogitTokens;
+  while (tile > 1 && experts * ((tokens + tile - 1) / tile) < 2048) tile /= 2;
   dim3 grid(static_cast<unsigned>((experts + kLogitWaves - 1) / kLogitWaves),
-            static_cast<unsigned>(token_tiles));
+            static_cast<unsigned>((tokens + tile - 1) / tile));
   if (weight_f32)
-    router_logits_kernel<2><<<grid, kLogitWaves * kWave, 0, as_stream(stream)>>>(x, w, logits, tokens,
-                                                                                experts, h);
+    router_logits_kernel<2><<<grid, kLogitWaves * kWave, 0, as_stream(stream)>>>(
+        x, w, logits, tokens, experts, h, tile);
   else
-    router_logits_kernel<1><<<grid, kLogitWaves * kWave, 0, as_stream(stream)>>>(x, w, logits, tokens,
-                                                                                experts, h);
+    router_logits_kernel<1><<<grid, kLogitWaves * kWave, 0, as_stream(stream)>>>(
+        x, w, logits, tokens, experts, h, tile);
   return check_launch("lk_router_logits");
 }
 
