@@ -272,8 +272,14 @@ LK_API int lk_w4a16_fused_qkv(const uint16_t* x, const uint8_t* q_packed,
  * weight decode's k order with its 128-wide group sums into the workspace and
  * the 64-row GEMM loads its rows from there straight into LDS. The workspace
  * holds lk_w4a16_dense_gemm_workspace(m, k, group) bytes (0 where that form
- * does not apply; -1 on bad input); a smaller one is refused before any launch. */
+ * does not apply; -1 on bad input); a smaller one is refused before any launch.
+ * With lk_dense_gemm_workspace(m, n, k, group, outputs, mxfp4) bytes (outputs:
+ * 3 for the fused QKV, else 1; mxfp4 != 0: lk_mxfp4_gemm_ws, group 32; never
+ * less than the query above) groups of 32 and 64 take that GEMM too, and a
+ * product too small to fill the GPU is split over k. */
 LK_API int64_t lk_w4a16_dense_gemm_workspace(int64_t m, int64_t k, int64_t group_size);
+LK_API int64_t lk_dense_gemm_workspace(int64_t m, int64_t n, int64_t k, int64_t group_size,
+                                       int64_t outputs, int mxfp4);
 LK_API int lk_w4a16_dense_gemm_ws(const uint16_t* x, const uint8_t* packed,
                                   const uint16_t* scales, uint16_t* y, int64_t m, int64_t n,
                                   int64_t k, int64_t group_size, void* workspace,
@@ -351,6 +357,10 @@ LK_API int lk_mxfp4_dequantise(const uint8_t* packed, const uint8_t* scale, void
  * engine/kernels/mxfp4_gemm.py:191-226. */
 LK_API int lk_mxfp4_gemm(const uint16_t* x, const uint8_t* packed, const uint8_t* scale,
                          uint16_t* y, int64_t m, int64_t n, int64_t k, int act_f16, void* stream);
+/* ... with an optional workspace of lk_dense_gemm_workspace() bytes. */
+LK_API int lk_mxfp4_gemm_ws(const uint16_t* x, const uint8_t* packed, const uint8_t* scale,
+                            uint16_t* y, int64_t m, int64_t n, int64_t k, int act_f16,
+                            void* workspace, int64_t workspace_bytes, void* stream);
 
 /* The same op as the reference variant: each weight decoded to the activation
  * type, then an fp32 dot, one thread per output

@@ -59,6 +59,7 @@ SIGNATURES: dict[str, list] = {
     "lk_mxfp4_quantise": [_P, _P, _P, _I64, _I64, _P],
     "lk_mxfp4_dequantise": [_P, _P, _P, _I64, _I64, _I, _P],
     "lk_mxfp4_gemm": [_P, _P, _P, _P, _I64, _I64, _I64, _I, _P],
+    "lk_mxfp4_gemm_ws": [_P, _P, _P, _P, _I64, _I64, _I64, _I, _P, _I64, _P],
     "lk_mxfp4_gemm_reference": [_P, _P, _P, _P, _I64, _I64, _I64, _I, _P],
     "lk_mxfp4_grouped_gemm": [_P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64, _P, _I64, _P],
     "lk_mxfp4_swiglu_gemm": [_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I64, _I64, _I64,
@@ -86,6 +87,7 @@ QUERIES: dict[str, list] = {
     "lk_w4a16_moe_decode_workspace": [_I64, _I64, _I64, _I64, _I64],
     "lk_w4a16_moe_forward_static_capacity": [],
     "lk_w4a16_dense_gemm_workspace": [_I64, _I64, _I64],
+    "lk_dense_gemm_workspace": [_I64, _I64, _I64, _I64, _I64, _I],
     "lk_w4a16_grouped_gemm_workspace": [_I64, _I64, _I64],
     "lk_w4a16_moe_forward_workspace": [_I64, _I64, _I64, _I64, _I64],
     "lk_mxfp4_moe_forward_workspace": [_I64, _I64, _I64, _I64, _I64],

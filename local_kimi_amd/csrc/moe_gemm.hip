@@ -28,23 +28,22 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <initializer_list>
 #include <mutex>
 
-#include "lk_common.hpp"
+#include "lk_gemm.hpp"
 #include "lk_route.hpp"
+#include "tile_gemm.hpp"
 
 namespace lk {
 namespace {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------
 // route schedule
 
 constexpr int kSchedThreads = 512;
 constexpr int kSchedWaves = kSchedThreads / kWave;
-constexpr int kTileRows = 64;       // rows per tile of the LDS-staged GEMM
 constexpr int kSmallTileRows = 16;  // rows per tile of the streaming GEMM
 constexpr int kMaxBuckets = 513;  // experts + 1 (the last bucket collects invalid routes)
 
@@ -314,244 +313,63 @@ schedule_one_kernel(const RouteTable rt, int64_t n, Schedule sc, const float* __
 // ---------------------------------------------------------------------------
 // W4A16 GEMM on the matrix cores
 
-// weight format x activation type; kFmtMxF8: MXFP4 weights x activations
-// split into fp8 hi + lo with per-32 E8M0 exponents (scaled fp4 MFMA)
-// kFmtW4G32 / kFmtW4G64: W4A16 with groups of 32 / 64 on 16-byte weight loads
-// (transpose4), in kernels whose kFmtW4A16 form takes G = 128 only
-enum : int { kFmtW4A16 = 0, kFmtMxBf16 = 1, kFmtMxF16 = 2, kFmtMxF8 = 3, kFmtW4G32 = 4, kFmtW4G64 = 5 };
-constexpr bool fmt_is_w4(int fmt) { return fmt == kFmtW4A16 || fmt == kFmtW4G32 || fmt == kFmtW4G64; }
-// group width of the 16-byte-load W4A16 forms, and their MFMAs (32 of k) per group
-constexpr int fmt_group(int fmt) { return fmt == kFmtW4G32 ? 32 : fmt == kFmtW4G64 ? 64 : 128; }
-constexpr int fmt_chain(int fmt) { return fmt_group(fmt) / 32; }
-enum : int { kActSwiglu = 0, kActSitu = 1 };                   // two-matrix epilogues
-
-struct GemmArgs {
-  const uint16_t* a;         // activations (bf16, or fp16 for kFmtMxF16), rows of k
-  const uint8_t* a_hi;       // kFmtMxF8: fp8 hi codes, rows of k bytes
-  const uint8_t* a_lo;       // kFmtMxF8: fp8 lo codes
-  const uint16_t* a_sc;      // kFmtMxF8: per-32 exponents, byte 0 hi, byte 1 lo
-  // 64-row expert-major launches with 128-wide k-steps (gate/up gather, down
-  // scatter; W4A16 G = 128 or MXFP4 on bf16 MFMA) load activations into LDS
-  // with direct loads: W4A16 from a_pair (rows of a with every 8-value chunk
-  // in the weight decode's k order) and a_neg (-136 * sum(x) per row and
-  // 128-wide group), MXFP4 from a. a_rows bounds both buffers.
-  const uint16_t* a_pair;
-  const float* a_neg;
-  int64_t a_rows;
-  // W4A16 gate/up on those launches: write the activations paired (the down
-  // GEMM's a_pair) and their group sums here (its a_neg); null: plain rows
-  float* out_neg;
-  const int32_t* perm;       // sorted position -> entry (gather / scatter modes)
-  const int32_t* tiles;      // [*, 4] tile list (schedule modes)
-  const int32_t* tile_count;
-  // the merged 64-row list of the same schedule (tails of <= 16 rows joined
-  // to the tile before them): what the direct-load launches walk
-  const int32_t* mtiles;
-  const int32_t* mtile_count;
-  const uint8_t* wp[3];      // packed weights per output matrix (two-matrix: gate, up)
-  const void* ws[3];         // scales: bf16 (W4A16) or E8M0 bytes (MXFP4)
-  uint16_t* out[3];
-  int64_t n, k, group;
-  int64_t wstride;           // packed bytes per expert
-  int64_t sstride;           // scale elements per expert
-  int64_t routes;            // entries per token (gather: token = entry / routes)
-  int dense_rows;            // rows of a dense product
-  int col_blocks;            // column blocks per output matrix
-  int outputs;               // output matrices (3 for fused QKV, else 1)
-  int act;                   // two-matrix epilogue (kActSwiglu / kActSitu)
-  int tail16;                // 64-row launches: tiles of <= 16 rows take the 16-row path
-  float situ_beta, situ_linear_beta;  // SiTU parameters; linear_beta <= 0: none
-  // persistent gate/up launches of small batches that route and schedule the
-  // batch themselves (no router or schedule launch before them): the
-  // router's inputs, the outputs block 0 writes, and the batch
-  const float* rt_logits;
-  const float* rt_bias;
-  int64_t* rt_idx;
-  float* rt_w;
-  int rt_tokens, rt_routed, rt_top_k, rt_renorm;
-  float rt_scaling;
-  // nonzero: the selections come from rt_idx (written by the router launch)
-  // and the block only ranks them
-  int rt_from_idx;
-  // where block 0 also writes the schedule (perm, tiles, count) for a later
-  // launch of the same block (the split SwiGLU's down GEMM); null: not needed
-  int32_t* rt_perm_out;
-  int32_t* rt_tiles_out;
-  int32_t* rt_count_out;
-};
-
-template <typename T>
-__device__ inline T pick3(const T (&v)[3], int i) {
-  return i == 0 ? v[0] : (i == 1 ? v[1] : v[2]);
-}
-
-constexpr int kSub = 4;       // 16-row MFMA subtiles per 64-row tile
 constexpr int kGemmWaves = 4;
-constexpr uint32_t kOnesBf16x2 = 0x3F803F80u;  // (1.0, 1.0) in bf16
 
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-typedef int v8i32_t __attribute__((ext_vector_type(8)));
-
-// ((w ^ 0x88888888) >> 4j) & 0x000F000F | 0x43004300 rewritten as
-// ((w >> 4j) & 0x000F000F) ^ 0x43084308: every nibble of the flip is 8 and the
-// flipped bit never overlaps the bf16 128.0 bits, so each output is one shift
-// and one three-input bit op.
-constexpr uint32_t kFlip128 = kBf16_128 | (kNibbleFlip & kPairMask);  // 0x43084308
-__device__ inline bf16x8_t unpack_q8(uint32_t w) {
-  const u32x4_t v = {(w & kPairMask) ^ kFlip128, ((w >> 4) & kPairMask) ^ kFlip128,
-                     ((w >> 8) & kPairMask) ^ kFlip128, ((w >> 12) & kPairMask) ^ kFlip128};
-  return __builtin_bit_cast(bf16x8_t, v);
-}
-
-// W4A16 groups narrower than a k-step on 16-byte loads: lane block jq = lane / 16
-// loads codes 32 jq .. 32 jq + 31 of its column, but an MFMA must stay inside
-// one group, so MFMA t takes codes 32 t .. 32 t + 31 and lane block jq needs
-// dword jq of block t: a 4 x 4 transpose over (dword, lane block), two
-// half-wave swaps and two row swaps. The four dwords loaded apart (and four
-// 2-byte scales) are eight loads a k-step instead of two: at 16 tokens of the
-// Kimi-Linear layer with G = 32 they held the block to 1.0 TB/s, 416 us with
-// its norms and router, against 147 us on the persistent kernel in this form.
-__device__ inline void transpose4(uint32_t (&w)[4]) {
-  auto half = [](uint32_t& a, uint32_t& b) {
-    const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
-    a = r[0];
-    b = r[1];
-  };
-  auto row = [](uint32_t& a, uint32_t& b) {
-    const auto r = __builtin_amdgcn_permlane16_swap(a, b, false, false);
-    a = r[0];
-    b = r[1];
-  };
-  half(w[0], w[2]);
-  half(w[1], w[3]);
-  row(w[0], w[1]);
-  row(w[2], w[3]);
-}
-
-// 2**(e - 127) as fp32 for an E8M0 byte (e = 0: the subnormal 2**-127, 255: inf)
-__device__ inline float e8m0_to_f32(uint32_t e) {
-  return __builtin_bit_cast(float, e == 0u ? 0x00400000u : e << 23);
-}
-
-// 8 E2M1 codes (natural order, low nibble first) times 2**(e - 127), exact in
-// bf16 / fp16 within range: the gfx950 scaled convert, two codes per byte.
-__device__ inline u32x4_t unpack_fp4x8_bf16(uint32_t w, float scale) {
-  const u32x4_t v = {
-      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 0)),
-      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 1)),
-      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 2)),
-      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 3))};
-  return v;
-}
-__device__ inline u32x4_t unpack_fp4x8_f16(uint32_t w, float scale) {
-  const u32x4_t v = {
-      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 0)),
-      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 1)),
-      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 2)),
-      __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 3))};
-  return v;
-}
-
-// K3's SiTU (engine/kernels/moe_grouped.py:163-178): gate and up rounded to
-// bf16 first (they are linear outputs), fp32 math, one rounding at the end.
-__device__ inline uint16_t situ_bf16(float gate_acc, float up_acc, float beta, float lbeta) {
-  const float g = round_bf16(gate_acc);
-  float u = round_bf16(up_acc);
-  const float ag = beta * tanhf(g / beta) * (1.0f / (1.0f + expf(-g)));
-  if (lbeta > 0.f) u = lbeta * tanhf(u / lbeta);
-  return f32_to_bf16(ag * u);
-}
-
-// fp32 sum of 8 bf16 activations: four dot2 against (1, 1), exact products
-__device__ inline float sum_x8_dot(const uint4 v) {
-  float s = dot2_bf16(v.x, kOnesBf16x2, 0.f);
-  s = dot2_bf16(v.y, kOnesBf16x2, s);
-  s = dot2_bf16(v.z, kOnesBf16x2, s);
-  return dot2_bf16(v.w, kOnesBf16x2, s);
-}
-
-// ---- direct global -> LDS loads (buffer_load ... lds)
-// One wave-wide load: lane L's 16 (or 4) bytes at voff + soff of the buffer
-// land in LDS at lds + 16 L (4 L); lds and soff are wave-uniform. Issued from
-// inline asm so that the compiler does not order LDS reads behind it: the
-// caller waits for it (s_waitcnt vmcnt) before the barrier that publishes
-// the LDS buffer, and the "memory" clobber keeps the loads issued after it
-// in program order (which that vmcnt count relies on).
-__device__ inline uint32_t lds_offset(const void* p) {
-  return static_cast<uint32_t>(
-      reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const char*)(p)));
-}
-// raw buffer descriptor of `bytes` bytes at `base` (stride 0; loads at or
-// past `bytes` return zeros)
-__device__ inline u32x4_t buffer_rsrc(const void* base, int64_t bytes) {
-  const uint64_t a = reinterpret_cast<uint64_t>(base);
-  const uint32_t n = bytes < 0xFFFFFFFFll ? static_cast<uint32_t>(bytes) : 0xFFFFFFFFu;
-  return u32x4_t{static_cast<uint32_t>(a), static_cast<uint32_t>(a >> 32) & 0xFFFFu, n,
-                 0x00020000u};
-}
-__device__ inline void lds_direct16(u32x4_t rs, const void* lds, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               ::"s"(__builtin_amdgcn_readfirstlane(lds_offset(lds))), "v"(voff), "s"(rs),
-                 "s"(__builtin_amdgcn_readfirstlane(soff))
-               : "memory");
-}
-__device__ inline void lds_direct4(u32x4_t rs, const void* lds, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-               ::"s"(__builtin_amdgcn_readfirstlane(lds_offset(lds))), "v"(voff), "s"(rs),
-                 "s"(__builtin_amdgcn_readfirstlane(soff))
-               : "memory");
-}
-
-// Rows of bf16 activations for the direct-load W4A16 GEMM: each 8-value chunk
+// Rows of bf16 activations for the direct-load W4A16 GEMMs: each 8-value chunk
 // in the weight decode's k order (x0 x4, x1 x5, x2 x6, x3 x7, as the
-// streaming kernel stages it) and -136 * sum(x) per 128-wide group, summed
-// in the staging's order: one 16-lane DPP row per (row, group), lane c on
-// chunk c, so the sums are bit-identical to the in-kernel staging's.
-// Unit u of the pairing (row u / (k / 128), group u % (k / 128)) by one
-// 16-lane row: lane c pairs chunk c and the row sums the group (live is
+// streaming kernel stages it) and -136 * sum(x) per group: one float per
+// 128-wide k-step at G = 128, four at G = 32 and 64 (CHAIN = 1, 2 MFMAs per
+// group; G = 64 fills the first of each pair). One 16-lane DPP row per (row,
+// k-step), lane c on chunk c, so the sums are bit-identical to the in-kernel
+// staging's.
+// Unit u of the pairing (row u / (k / 128), k-step u % (k / 128)) by one
+// 16-lane row: lane c pairs chunk c and the row sums the groups (live is
 // uniform over the row; a dead row loads unit 0 and stores nothing).
+template <int CHAIN>
 __device__ inline void pair_unit(const uint16_t* __restrict__ x, uint16_t* __restrict__ xp,
                                  float* __restrict__ neg, uint32_t unit, bool live) {
   const uint32_t u = live ? unit : 0u;
-  const int64_t off = static_cast<int64_t>(u) * 128 + (threadIdx.x & 15) * 8;
+  const int c = threadIdx.x & 15;
+  const int64_t off = static_cast<int64_t>(u) * 128 + c * 8;
   const uint4 v = *reinterpret_cast<const uint4*>(x + off);
   uint32_t q[4];
   pair_x8(v, q);
-  float sx = sum8(sum_x8_dot(v));
-  sx += dpp_f32<kRowMirror>(sx);
+  const float sx = pair_group_sum<CHAIN>(v);
   if (live) {
     *reinterpret_cast<uint4*>(xp + off) = make_uint4(q[0], q[1], q[2], q[3]);
-    if ((threadIdx.x & 15) == 0) neg[u] = -kCodeOffset * sx;
+    if ((c & (4 * CHAIN - 1)) == 0)
+      neg[CHAIN == 4 ? u : 4 * static_cast<int64_t>(u) + c / 4] = -kCodeOffset * sx;
   }
 }
 
+template <int CHAIN>
 __global__ void __launch_bounds__(256)
 pair_rows_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ xp,
                  float* __restrict__ neg, uint32_t units) {
-  // unit = row * (k / 128) + group, so its chunk sits at 128 unit + 8 c
+  // unit = row * (k / 128) + k-step, so its chunk sits at 128 unit + 8 c
   const uint32_t unit = (blockIdx.x * 256u + threadIdx.x) >> 4;
-  pair_unit(x, xp, neg, unit, unit < units);  // uniform over each 16-lane row
+  pair_unit<CHAIN>(x, xp, neg, unit, unit < units);  // uniform over each 16-lane row
 }
 
 // The router and the activation pairing of a prefill-sized batch in one
 // launch: block t routes token t in its first wave (route_token, as the
 // router kernel does: engine/klinear/router.py:47-85) and pairs token t's
-// k / 128 groups in its 16-lane rows (pair_unit, as pair_rows_kernel does),
+// k / 128 k-steps in its 16-lane rows (pair_unit, as pair_rows_kernel does),
 // so the selections, weights and paired rows are those two launches' bits.
 constexpr int kRoutePairThreads = 320;
 
-template <int EPL>
+template <int EPL, int CHAIN>
 __global__ void __launch_bounds__(kRoutePairThreads)
 route_pair_kernel(const float* __restrict__ logits, const float* __restrict__ bias,
                   int64_t* __restrict__ idx, float* __restrict__ w, int experts, int top_k,
                   float scaling, int renorm, const uint16_t* __restrict__ x,
-                  uint16_t* __restrict__ xp, float* __restrict__ neg, int groups) {
+                  uint16_t* __restrict__ xp, float* __restrict__ neg, int steps) {
   const int64_t t = blockIdx.x;
   if (threadIdx.x < kWave)
     route_token<EPL>(logits + t * experts, bias, experts, top_k, -1, scaling, renorm,
                      idx + t * top_k, w + t * top_k);
-  for (int gq = threadIdx.x >> 4; gq < groups; gq += kRoutePairThreads / 16)  // per 16-lane row
-    pair_unit(x, xp, neg, static_cast<uint32_t>(t * groups + gq), true);
+  for (int q = threadIdx.x >> 4; q < steps; q += kRoutePairThreads / 16)  // per 16-lane row
+    pair_unit<CHAIN>(x, xp, neg, static_cast<uint32_t>(t * steps + q), true);
 }
 
 // Zero line read by ring reloads past the last k-step. Every wave reads the
@@ -952,13 +770,6 @@ constexpr int kStWaves = 8;
 constexpr int kStDepth = 6;                      // k-steps of weights in flight per wave
 constexpr int kStMaxLds = 150 * 1024;            // LDS a streaming block may take
 constexpr int kStPassSteps = 4;                  // k-steps per activation pass (64-row tiles)
-constexpr int64_t kMaxDirectBytes = 0xFFFFFFFFll;  // direct-load sources: 32-bit byte offsets
-
-template <int FMT>
-__device__ inline uint16_t store_value(float v) {
-  if constexpr (FMT == kFmtMxF16) return __builtin_bit_cast(uint16_t, static_cast<_Float16>(v));
-  else return f32_to_bf16(v);
-}
 
 // LDS bytes of one streaming block with 16 * mt-row tiles: mt == 1 keeps all
 // k-steps of the tile's activations (one buffer); mt > 1 double-buffers
@@ -971,24 +782,10 @@ inline size_t stream_lds_bytes(int64_t k, int mt) {
   return static_cast<size_t>(nbuf * ps * mt) * (4 * kWave * sizeof(uint4) + 4 * 16 * sizeof(float));
 }
 
-// s_waitcnt vmcnt(N) from inline asm (the compiler does not count the
-// direct loads, so it cannot place this wait itself)
-template <int N>
-__device__ inline void wait_vmcnt() {
-  static_assert(N >= 0 && N <= 63, "vmcnt range");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
-// Slot swizzle of row m in the direct-load activation layout: (m & 15) with
-// its two 2-bit halves swapped.
-__device__ inline int row_swizzle(int m) { return ((m >> 2) & 3) | ((m & 3) << 2); }
-
 // One tile of <= 16 * MT rows x kBN columns of a streaming block (below).
-// MT = 1: all k-steps of the activations resident; MT = 4 or 5: passes of
-// kStPassSteps (5: 3) k-steps, double buffered. DIRECT: activations come in by
-// direct loads (see GemmArgs::a_pair).
-template <int FMT, int MATS, int NT, int MT, bool WIDE, bool GATHER, bool SCATTER, bool DENSE,
-          bool DIRECT = false>
+// MT = 1: all k-steps of the activations resident; MT = 4: passes of
+// kStPassSteps k-steps, double buffered.
+template <int FMT, int MATS, int NT, int MT, bool WIDE, bool GATHER, bool SCATTER, bool DENSE>
 __device__ __forceinline__ void stream_tile(const GemmArgs& g, const int expert, const int row0,
                                             const int rows, const int cb, const int osel) {
   constexpr bool kMx = FMT != kFmtW4A16;
@@ -999,14 +796,9 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& g, const int expert,
   constexpr int kBN = kStWaves * NT * 16;
   constexpr int kRows = 16 * MT;
   constexpr int kNBuf = MT == 1 ? 1 : 2;
-  constexpr int kPS = MT == 5 ? 3 : kStPassSteps;  // k-steps per pass (MT > 1)
+  constexpr int kPS = kStPassSteps;  // k-steps per pass (MT > 1)
   constexpr int kPassUnits = MT == 1 ? 1 : (kRows * kPS * 16 + kThreads - 1) / kThreads;
-  constexpr bool kDirect = DIRECT;
-  static_assert(!kDirect || (WIDE && (FMT == kFmtW4A16 || FMT == kFmtMxBf16) &&
-                             (DENSE ? !GATHER && !SCATTER : GATHER != SCATTER)),
-                "direct loads: 128-wide k-steps of a dense product or an expert-major gather "
-                "or scatter");
-  static_assert(MT == 1 || MT == 4 || (MT == 5 && kDirect), "tile heights 16, 64, direct 80");
+  static_assert(MT == 1 || MT == 4, "tile heights 16, 64");
   extern __shared__ uint4 smem[];
   __shared__ int64_t row_index[kRows];  // activation row of each tile row
   __shared__ int64_t out_row[kRows];    // output row of each tile row
@@ -1015,12 +807,9 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& g, const int expert,
   const int tid = threadIdx.x;
 
   // the tile's sorted-position lookups, issued ahead of the weight loads so
-  // that waiting for them never waits for weights. Direct loads fill every
-  // tile row: rows past `rows` read the tile's first row (never stored).
-  const int table_rows = kDirect ? kRows : rows;
-  const int src_m = kDirect && tid >= rows ? 0 : tid;
+  // that waiting for them never waits for weights
   int32_t pos = 0;
-  if ((GATHER || SCATTER) && tid < table_rows) pos = g.perm[row0 + src_m];
+  if ((GATHER || SCATTER) && tid < rows) pos = g.perm[row0 + tid];
   const int lane = tid & (kWave - 1);
   const int wv = tid / kWave;
   const int jq = lane >> 4;
@@ -1069,8 +858,8 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& g, const int expert,
 
   // 2. the tile's activation and output rows (one lookup per row, shared
   // through LDS; the epilogue then reads no global memory)
-  if (tid < table_rows) {
-    row_index[tid] = GATHER ? static_cast<int64_t>(pos / g.routes) : row0 + src_m;
+  if (tid < rows) {
+    row_index[tid] = GATHER ? static_cast<int64_t>(pos / g.routes) : row0 + tid;
     out_row[tid] = SCATTER ? static_cast<int64_t>(pos) : row0 + tid;
   }
   __syncthreads();
@@ -1079,7 +868,7 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& g, const int expert,
   // units of one (row, step) sit in one 16-lane DPP row; slots m >= rows are
   // skipped (their MFMA rows are never stored)
   constexpr int kRowShift = MT == 1 ? 4 : 6;
-  static_assert(kDirect || kRows == (1 << kRowShift), "staged tiles have 16 or 64 rows");
+  static_assert(kRows == (1 << kRowShift), "tiles have 16 or 64 rows");
   auto unit_live = [&](int u) { return ((u >> 4) & (kRows - 1)) < rows; };
   // kFmtMxF8: unit c < 8 is 16 fp8 hi codes (k = 16c..16c+15 of the step),
   // c >= 8 the lo codes of chunk c - 8; units c < 4 also carry the row's
@@ -1143,95 +932,10 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& g, const int expert,
   };
   auto pass_steps = [&](int p) { return min(ps, ksteps - p * ps); };
 
-  // Direct-load layout: a k-step's activations are [tile row m][slot] of 16
-  // bytes, chunk c (k = 8c..8c+7 of the step) of row m in slot c ^ rs(m),
-  // rs(m) = (m & 15) with its two 2-bit halves swapped, so 16 lanes of one
-  // load read one row's 256 contiguous bytes and an MFMA fragment read (16
-  // rows, one chunk each) is free of bank conflicts (measured by the
-  // SQ_LDS_BANK_CONFLICT counter on this access pattern: the plain c ^ (m & 15)
-  // costs 4 conflict cycles per 16-byte read, this one none). One load
-  // fills a block of 4 rows of one k-step (lane L: row 4 blk + L / 16, chunk
-  // (L & 15) ^ (row & 15)). MT > 1: wave wv fills blocks wv, wv + 8, ... of
-  // every k-step of a pass. MT == 1 (one pass over all k-steps): wave wv
-  // fills block wv & 3 of k-steps wv / 4, wv / 4 + 2, ...
-  // W4A16's group sums come in by 4-byte loads of 64 tile rows (lane = row;
-  // lanes past the tile read row 0 into padding) to offs[buffer][ls][row]:
-  // MT > 1: wave n loads step n / kNegLoads, rows 64 (n % kNegLoads) ..;
-  // MT == 1: waves take the steps round robin.
-  // MT > 1: a wave issues its direct loads before its kPS steps of weight
-  // refills (2 MATS NT loads each), so vmcnt(kAfter) at the pass end covers
-  // them; MT == 1 issues them after the ring and waits for everything.
-  constexpr int kBlocks = kRows / 4;                                      // per k-step
-  constexpr int kPw = MT == 1 ? 1 : (kBlocks + kStWaves - 1) / kStWaves;  // blocks per wave
-  constexpr int kNegLoads = (kRows + 63) / 64;                            // per k-step
-  constexpr int kNegStride = kNegLoads * 64;                              // floats per k-step
-  constexpr int kAfter = kPS * 2 * MATS * NT;
-  static_assert(!kDirect || MT == 1 || kPS * kNegLoads <= kStWaves, "one sum load per wave");
-  static_assert(kNegLoads <= 2, "at most 128 tile rows");
-  [[maybe_unused]] uint32_t voff[kPw] = {};
-  [[maybe_unused]] uint32_t voff_neg0 = 0, voff_neg1 = 0;  // rows lane, 64 + lane
-  [[maybe_unused]] u32x4_t rs_a = {0u, 0u, 0u, 0u}, rs_n = {0u, 0u, 0u, 0u};
-  if constexpr (kDirect) {
-    rs_a = buffer_rsrc(FMT == kFmtW4A16 ? g.a_pair : g.a, g.a_rows * K * 2);
-#pragma unroll
-    for (int h = 0; h < kPw; ++h) {
-      const int blk = MT == 1 ? (wv & 3) : min(wv + kStWaves * h, kBlocks - 1);
-      const int m = blk * 4 + jq;
-      voff[h] = static_cast<uint32_t>(row_index[m] * K * 2 + ((lane & 15) ^ row_swizzle(m)) * 16);
-    }
-    if constexpr (FMT == kFmtW4A16) {
-      rs_n = buffer_rsrc(g.a_neg, g.a_rows * (K / 128) * 4);
-      voff_neg0 = static_cast<uint32_t>(row_index[lane < kRows ? lane : 0] * (K / 128) * 4);
-      if constexpr (kNegLoads > 1)
-        voff_neg1 = static_cast<uint32_t>(row_index[64 + lane < kRows ? 64 + lane : 0] * (K / 128) * 4);
-    }
-  }
-  auto direct_pass = [&](int p, int b) {
-    if constexpr (kDirect) {
-      const int steps = pass_steps(p);
-      if constexpr (MT == 1) {
-        for (int ls = wv >> 2; ls < steps; ls += 2)
-          lds_direct16(rs_a, afrag + (ls * kRows + (wv & 3) * 4) * 16, voff[0],
-                       static_cast<uint32_t>(ls) * 256u);
-        if constexpr (FMT == kFmtW4A16) {
-          for (int ls = wv; ls < steps; ls += kStWaves)
-            lds_direct4(rs_n, offs + ls * kNegStride, voff_neg0, static_cast<uint32_t>(ls) * 4u);
-        }
-      } else {
-#pragma unroll
-        for (int h = 0; h < kPw; ++h) {
-          const int blk = wv + kStWaves * h;
-          if (blk < kBlocks) {
-#pragma unroll
-            for (int ls = 0; ls < kPS; ++ls)
-              if (ls < steps)
-                lds_direct16(rs_a, afrag + ((b * ps + ls) * kRows + blk * 4) * 16, voff[h],
-                             static_cast<uint32_t>(p * ps + ls) * 256u);
-          }
-        }
-        if constexpr (FMT == kFmtW4A16) {
-          const int ls = wv / kNegLoads, hh = wv % kNegLoads;
-          if (ls < steps)
-            lds_direct4(rs_n, offs + (b * ps + ls) * kNegStride + hh * 64,
-                        hh == 0 ? voff_neg0 : voff_neg1,
-                        static_cast<uint32_t>(p * ps + ls) * 4u);
-        }
-      }
-    }
-  };
-
   // 3. stage the first pass. 64-row tiles: all of its units in one batch of
   // loads, then the weight ring, then the stores (the stores wait for the
-  // activation loads alone); direct loads: the pass, then the ring
-  if constexpr (kDirect && MT == 1) {
-    direct_pass(0, 0);  // the ring is already in flight
-    wait_vmcnt<0>();
-  } else if constexpr (kDirect) {
-    direct_pass(0, 0);
-#pragma unroll
-    for (int j = 0; j < kRing; ++j) w[j].load(wrow, srow, j, jq, K, gshift, ksteps, dummy);
-    wait_vmcnt<kAfter>();
-  } else if constexpr (MT > 1) {
+  // activation loads alone)
+  if constexpr (MT > 1) {
     uint4 v0[kPassUnits];
     uint32_t s0[kPassUnits];
     const int units0 = pass_steps(0) * kRows * 16;
@@ -1287,13 +991,9 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& g, const int expert,
         acc[mi][nt][ms] = zero4;
       }
   // LDS slot of this lane's MFMA fragment (subtile ms, sub-step t) of local
-  // k-step ls in buffer b: the swizzled fragment blocks of the staged layout,
-  // or the row-major layout of direct loads (this lane's row within a subtile
-  // is ln, so its swizzle is rs(ln))
-  [[maybe_unused]] const int rsw = row_swizzle(ln);
+  // k-step ls in buffer b
   auto a_slot = [&](int b, int ls, int ms, int t) -> int {
-    if constexpr (kDirect) return ((b * ps + ls) * kRows + ms * 16 + ln) * 16 + ((4 * jq + t) ^ rsw);
-    else return (((b * ps + ls) * MT + ms) * 4 + t) * kWave + jq * 16 + (ln ^ (4 * t + jq));
+    return (((b * ps + ls) * MT + ms) * 4 + t) * kWave + jq * 16 + (ln ^ (4 * t + jq));
   };
   // one k-step: weights wj (a ring slot), activation buffer b, local step ls.
   // Every subtile is computed (no per-MFMA branch): rows past the tile read
@@ -1394,8 +1094,7 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& g, const int expert,
 #pragma unroll
       for (int ms = 0; ms < MT; ++ms)
         neg[ms] = *reinterpret_cast<const f32x4_t*>(
-            &offs[kDirect ? (b * ps + ls) * kNegStride + ms * 16 + jq * 4
-                          : (frag0 + ms * 4) * 16 + jq * 4]);
+            &offs[(frag0 + ms * 4) * 16 + jq * 4]);
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
         bf16x8_t af[MT];
@@ -1470,7 +1169,7 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& g, const int expert,
       }
     }
   } else {
-    // 64- and 80-row tiles: passes of kPS k-steps; the ring is one pass deep
+    // 64-row tiles: passes of kPS k-steps; the ring is one pass deep
     // (its first kPS slots), so slot j serves local step j
     // No exit inside a pass (see the 16-row loop): a partial last pass skips
     // the compute of its missing steps only.
@@ -1481,10 +1180,7 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& g, const int expert,
       const int b = p % kNBuf;
       const bool more = p + 1 < passes;
       const int units1 = more ? pass_steps(p + 1) * kRows * 16 : 0;
-      if constexpr (kDirect) {
-        // the next pass's buffer was retired by the previous pass's barrier
-        if (more) direct_pass(p + 1, (p + 1) % kNBuf);
-      } else if (more) {
+      if (more) {
 #pragma unroll
         for (int q = 0; q < kPassUnits; ++q) {
           const int u = q * kThreads + tid;
@@ -1503,14 +1199,10 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& g, const int expert,
       if (more) {
         // publish the next pass; the barrier also retires this pass's buffer,
         // which the pass after next overwrites
-        if constexpr (kDirect) {
-          wait_vmcnt<kAfter>();  // this wave's direct loads landed
-        } else {
 #pragma unroll
-          for (int q = 0; q < kPassUnits; ++q) {
-            const int u = q * kThreads + tid;
-            if (u < units1 && unit_live(u)) unit_store((p + 1) % kNBuf, u, vnext[q], snext[q]);
-          }
+        for (int q = 0; q < kPassUnits; ++q) {
+          const int u = q * kThreads + tid;
+          if (u < units1 && unit_live(u)) unit_store((p + 1) % kNBuf, u, vnext[q], snext[q]);
         }
         __syncthreads();
       }
@@ -1525,64 +1217,18 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& g, const int expert,
     else
       return store_value<FMT>(tot[0][nt][ms][i]);
   };
-  if constexpr (kDirect) {
-    // the tile goes through LDS ([row][column], rows padded by 8 values so
-    // that the 2-byte writes of 4 rows spread over the banks) and out as
-    // 16-byte chunks, a row's block columns contiguous. W4A16 gate/up with
-    // out_neg: each chunk paired and the 128-wide group sums written too, in
-    // the staging's order (the block's kBN = 128 columns are one group; the
-    // 16 chunks of a row sit in one 16-lane DPP row).
-    constexpr int kPitch = kBN + 8;
-    constexpr int kChunks = kBN / 8;
-    static_assert(kChunks % 16 == 0 && kThreads % 16 == 0, "chunks of a row fill DPP rows");
-    uint16_t* const otile = reinterpret_cast<uint16_t*>(smem);
-    __syncthreads();  // every wave has read its last activations
 #pragma unroll
-    for (int ms = 0; ms < MT; ++ms) {
-      if (ms >= mt_act) break;
+  for (int ms = 0; ms < MT; ++ms) {
+    if (ms >= mt_act) break;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 4; ++i) {
+      const int m = ms * 16 + jq * 4 + i;
+      if (m >= rows) continue;
+      const int64_t orow = out_row[m];
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt)
-          otile[(ms * 16 + jq * 4 + i) * kPitch + (wv * NT + nt) * 16 + ln] = out_value(nt, ms, i);
-    }
-    __syncthreads();
-    constexpr bool kPairOut = FMT == kFmtW4A16 && MATS == 2;
-    static_assert(!kPairOut || kBN == 128, "paired output: one group per block");
-    for (int u = tid; u < kRows * kChunks; u += kThreads) {
-      const int m = u / kChunks, c = u - m * kChunks;
-      const uint4 v = *reinterpret_cast<const uint4*>(otile + m * kPitch + c * 8);
-      const int64_t c0 = static_cast<int64_t>(cb) * kBN + c * 8;
-      const bool live = m < rows && c0 < N;
-      if constexpr (kPairOut) {
-        if (g.out_neg) {
-          uint32_t q[4];
-          pair_x8(v, q);
-          float sx = sum8(sum_x8_dot(v));
-          sx += dpp_f32<kRowMirror>(sx);
-          if (live) {
-            *reinterpret_cast<uint4*>(out + out_row[m] * N + c0) = make_uint4(q[0], q[1], q[2], q[3]);
-            if (c == 0) g.out_neg[out_row[m] * (N / 128) + cb] = -kCodeOffset * sx;
-          }
-          continue;
-        }
-      }
-      if (live) *reinterpret_cast<uint4*>(out + out_row[m] * N + c0) = v;
-    }
-  } else {
-#pragma unroll
-    for (int ms = 0; ms < MT; ++ms) {
-      if (ms >= mt_act) break;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int m = ms * 16 + jq * 4 + i;
-        if (m >= rows) continue;
-        const int64_t orow = out_row[m];
-#pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-          if (col[nt] >= N) continue;
-          out[orow * N + col[nt]] = out_value(nt, ms, i);
-        }
+      for (int nt = 0; nt < NT; ++nt) {
+        if (col[nt] >= N) continue;
+        out[orow * N + col[nt]] = out_value(nt, ms, i);
       }
     }
   }
@@ -1594,8 +1240,7 @@ __device__ __forceinline__ void stream_tile(const GemmArgs& g, const int expert,
 // double buffered, the next pass loaded while the current one computes, one
 // barrier per pass); every wave streams its own columns over all of k with
 // kStDepth k-steps of weights in flight and stores its outputs itself.
-template <int FMT, int MATS, int NT, int MT, bool WIDE, bool GATHER, bool SCATTER, bool DENSE,
-          bool DDIRECT = false>
+template <int FMT, int MATS, int NT, int MT, bool WIDE, bool GATHER, bool SCATTER, bool DENSE>
 __global__ void __launch_bounds__(kStWaves * kWave, 2)
 w4a16_stream_kernel(const GemmArgs g) {
   constexpr int kThreads = kStWaves * kWave;
@@ -1652,35 +1297,16 @@ w4a16_stream_kernel(const GemmArgs g) {
     }
     return;
   }
-  // 64-row gather / scatter launches with 128-wide k-steps take their
-  // activations by direct loads, in every tile path below
-  // (DDIRECT: a dense product whose rows are loaded directly, W4A16 from the
-  // paired copy)
-  constexpr bool kDirect = MT > 1 && WIDE && (FMT == kFmtW4A16 || FMT == kFmtMxBf16) &&
-                           (DENSE ? DDIRECT : GATHER != SCATTER);
-  if constexpr (kDirect) {
-    // the merged list: an expert's last tile of <= 16 rows is already part of
-    // the 64-row tile before it, one pass over the expert's weights for up to
-    // 80 rows (and every entry of the list is a tile with rows to compute, so
-    // consecutive entries, which go to consecutive XCDs, carry equal work)
-    if (rows > 64) {
-      stream_tile<FMT, MATS, NT, 5, WIDE, GATHER, SCATTER, DENSE, true>(g, expert, row0, rows, cb,
-                                                                        osel);
-      return;
-    }
-  }
   // a tile of at most 16 rows (an expert's last rows) takes the 16-row path:
   // a quarter of the MFMAs and all of its activations resident (the host
   // sets tail16 when they fit the launch's LDS)
   if constexpr (MT > 1) {
     if (rows <= 16 && g.tail16) {
-      stream_tile<FMT, MATS, NT, 1, WIDE, GATHER, SCATTER, DENSE, kDirect>(g, expert, row0, rows,
-                                                                           cb, osel);
+      stream_tile<FMT, MATS, NT, 1, WIDE, GATHER, SCATTER, DENSE>(g, expert, row0, rows, cb, osel);
       return;
     }
   }
-  stream_tile<FMT, MATS, NT, MT, WIDE, GATHER, SCATTER, DENSE, kDirect>(g, expert, row0, rows, cb,
-                                                                        osel);
+  stream_tile<FMT, MATS, NT, MT, WIDE, GATHER, SCATTER, DENSE>(g, expert, row0, rows, cb, osel);
 }
 
 // ---------------------------------------------------------------------------
@@ -2700,9 +2326,9 @@ MoeLayout moe_layout(int64_t entries, int64_t experts, int64_t act_cols, int64_t
   l.x_pair = at;
   if (pairs) at += align_up(static_cast<size_t>(pair_rows) * out_cols * 2);
   l.x_neg = at;
-  if (pairs) at += align_up(static_cast<size_t>(pair_rows) * (out_cols / 128) * 4);
+  if (pairs) at += align_up(static_cast<size_t>(pair_rows) * (out_cols / 128) * 16);
   l.act_neg = at;
-  if (pairs) at += align_up(static_cast<size_t>(entries) * (act_cols / 128) * 4);
+  if (pairs) at += align_up(static_cast<size_t>(entries) * (act_cols / 128) * 16);
   l.total = at;
   return l;
 }
@@ -2768,12 +2394,15 @@ int schedule_launch(const RouteTable& rt, int64_t entries, char* ws, const Sched
 // Paired copy + group sums of `rows` bf16 rows of k (k % 128 == 0) for the
 // direct-load W4A16 GEMM.
 int pair_rows_launch(const uint16_t* x, uint16_t* xp, float* neg, int64_t rows, int64_t k,
-                     hipStream_t s) {
+                     int64_t group, hipStream_t s) {
   const int64_t units = rows * (k / 128);
   if (units == 0) return LK_OK;
   LK_REQUIRE(k % 128 == 0 && units < (1LL << 27), "pairing: unsupported size");
-  pair_rows_kernel<<<static_cast<unsigned>((units + 15) / 16), 256, 0, s>>>(
-      x, xp, neg, static_cast<uint32_t>(units));
+  const unsigned nb = static_cast<unsigned>((units * 16 + 255) / 256);
+  const uint32_t n = static_cast<uint32_t>(units);
+  if (group == 32) pair_rows_kernel<1><<<nb, 256, 0, s>>>(x, xp, neg, n);
+  else if (group == 64) pair_rows_kernel<2><<<nb, 256, 0, s>>>(x, xp, neg, n);
+  else pair_rows_kernel<4><<<nb, 256, 0, s>>>(x, xp, neg, n);
   return check_launch("moe activation pairing");
 }
 
@@ -2781,17 +2410,19 @@ int pair_rows_launch(const uint16_t* x, uint16_t* xp, float* neg, int64_t rows, 
 // routed experts; validated by the caller)
 int route_pair_launch(const float* logits, const float* bias, int64_t* idx, float* w,
                       int64_t tokens, int64_t routed, int64_t top_k, float scaling, int renorm,
-                      const uint16_t* x, uint16_t* xp, float* neg, int64_t k, hipStream_t s) {
+                      const uint16_t* x, uint16_t* xp, float* neg, int64_t k, int64_t group,
+                      hipStream_t s) {
   LK_REQUIRE(k % 128 == 0 && tokens * (k / 128) < (1LL << 27) && routed <= 256 &&
                  tokens <= 2147483647LL,
              "router + pairing: unsupported size");
-  route_pair_kernel<4><<<static_cast<unsigned>(tokens), kRoutePairThreads, 0, s>>>(
+  auto* fn = group == 32   ? &route_pair_kernel<4, 1>
+             : group == 64 ? &route_pair_kernel<4, 2>
+                           : &route_pair_kernel<4, 4>;
+  fn<<<static_cast<unsigned>(tokens), kRoutePairThreads, 0, s>>>(
       logits, bias, idx, w, static_cast<int>(routed), static_cast<int>(top_k), scaling, renorm,
       x, xp, neg, static_cast<int>(k / 128));
   return check_launch("moe router + activation pairing");
 }
-
-enum class Mode { Gather, Scatter, GatherScatter, Dense };
 
 template <int FMT, int MATS, int NT, bool WIDE>
 void gemm_dispatch_mode(const GemmArgs& g, Mode mode, unsigned blocks, hipStream_t s) {
@@ -2854,11 +2485,10 @@ int gemm_launch(GemmArgs g, Mode mode, int64_t tiles, bool wide_cols, hipStream_
   return check_launch(what);
 }
 
-template <int FMT, int MATS, int MT, bool WIDE, bool GATHER, bool SCATTER, bool DENSE,
-          bool DDIRECT = false>
+template <int FMT, int MATS, int MT, bool WIDE, bool GATHER, bool SCATTER, bool DENSE>
 void stream_one(const GemmArgs& g, unsigned blocks, size_t lds, hipStream_t s) {
   constexpr int NT = MATS == 2 ? 1 : 2;
-  auto* fn = &w4a16_stream_kernel<FMT, MATS, NT, MT, WIDE, GATHER, SCATTER, DENSE, DDIRECT>;
+  auto* fn = &w4a16_stream_kernel<FMT, MATS, NT, MT, WIDE, GATHER, SCATTER, DENSE>;
   static bool limit_set = false;  // the attribute is per function; set once per process
   if (!limit_set) {
     (void)hipFuncSetAttribute(reinterpret_cast<const void*>(fn),
@@ -2872,8 +2502,7 @@ void stream_one(const GemmArgs& g, unsigned blocks, size_t lds, hipStream_t s) {
 bool persist_disabled() { return path_choice(kKnobMoePersist) == 1; }
 
 template <int FMT, int MATS, int MT, bool WIDE>
-void stream_dispatch(const GemmArgs& g, Mode mode, unsigned blocks, size_t lds, hipStream_t s,
-                     bool dense_direct = false) {
+void stream_dispatch(const GemmArgs& g, Mode mode, unsigned blocks, size_t lds, hipStream_t s) {
   if constexpr (FMT == kFmtMxF16) {
     stream_one<FMT, MATS, MT, false, false, false, true>(g, blocks, lds, s);
   } else {
@@ -2884,12 +2513,6 @@ void stream_dispatch(const GemmArgs& g, Mode mode, unsigned blocks, size_t lds, 
         stream_one<FMT, MATS, MT, WIDE, true, true, false>(g, blocks, lds, s);
         break;
       case Mode::Dense:
-        if constexpr (MT > 1 && WIDE && (FMT == kFmtW4A16 || FMT == kFmtMxBf16)) {
-          if (dense_direct) {
-            stream_one<FMT, MATS, MT, WIDE, false, false, true, true>(g, blocks, lds, s);
-            break;
-          }
-        }
         stream_one<FMT, MATS, MT, WIDE, false, false, true>(g, blocks, lds, s);
         break;
     }
@@ -3089,25 +2712,6 @@ int stream_launch(GemmArgs g, Mode mode, int64_t tiles, int mt, hipStream_t s, c
   // 64-row launches: tiles of <= 16 rows run the 16-row path when all of
   // their activations fit the LDS the launch takes anyway
   g.tail16 = mt > 1 && stream_lds_bytes(g.k, 1) <= lds ? 1 : 0;
-  // 64-row gather / scatter launches load activations directly (byte
-  // offsets of 32 bits; W4A16 from the paired copy)
-  if (mt > 1 && wide && FMT != kFmtMxF8 && (mode == Mode::Gather || mode == Mode::Scatter)) {
-    LK_REQUIRE(g.a_rows > 0 && g.a_rows * g.k * 2 <= static_cast<int64_t>(kMaxDirectBytes),
-               "%s: activations out of range for direct loads", what);
-    LK_REQUIRE(FMT != kFmtW4A16 || (g.a_pair && g.a_neg), "%s: paired activations missing", what);
-    LK_REQUIRE(g.n % 8 == 0 && (!g.out_neg || (MATS == 2 && g.n % 128 == 0)),
-               "%s: output width %lld unsupported for direct loads", what, (long long)g.n);
-    LK_REQUIRE(g.mtiles && g.mtile_count, "%s: merged tile list missing", what);
-    g.tiles = g.mtiles;
-    g.tile_count = g.mtile_count;
-  }
-  // dense 64-row launches load their rows directly as well when they can:
-  // MXFP4 from the rows themselves, W4A16 from a paired copy with its group
-  // sums (a_pair / a_neg, made by the caller's pre-pass)
-  const bool dense_direct = mt > 1 && wide && mode == Mode::Dense && g.n % 8 == 0 &&
-                            g.a_rows > 0 &&
-                            g.a_rows * g.k * 2 <= static_cast<int64_t>(kMaxDirectBytes) &&
-                            (FMT == kFmtMxBf16 || (FMT == kFmtW4A16 && g.a_pair && g.a_neg));
   g.col_blocks = static_cast<int>((g.n + kStWaves * NT * 16 - 1) / (kStWaves * NT * 16));
   const int64_t blocks = (tiles + 7) / 8 * 8 * g.col_blocks * g.outputs;
   LK_REQUIRE(blocks > 0 && blocks < (1LL << 31), "%s: too many blocks", what);
@@ -3124,7 +2728,7 @@ int stream_launch(GemmArgs g, Mode mode, int64_t tiles, int mt, hipStream_t s, c
     if (wide) stream_dispatch<FMT, MATS, 1, kWideOk>(g, mode, nb, lds, s);
     else stream_dispatch<FMT, MATS, 1, false>(g, mode, nb, lds, s);
   } else {
-    if (wide) stream_dispatch<FMT, MATS, 4, kWideOk>(g, mode, nb, lds, s, dense_direct);
+    if (wide) stream_dispatch<FMT, MATS, 4, kWideOk>(g, mode, nb, lds, s);
     else stream_dispatch<FMT, MATS, 4, false>(g, mode, nb, lds, s);
   }
   return check_launch(what);
@@ -3132,6 +2736,36 @@ int stream_launch(GemmArgs g, Mode mode, int64_t tiles, int mt, hipStream_t s, c
 
 // Wider column blocks once there are enough tiles to fill the machine.
 bool wide_cols_for(int64_t tiles, int64_t n) { return tiles * ((n + 63) / 64) >= 2048; }
+
+// The prefill GEMM's format of a weight format and group width, -1 if it has none.
+int tile_format(int fmt, int64_t group) {
+  if (fmt != kFmtW4A16) return fmt == kFmtMxBf16 || fmt == kFmtMxF16 ? fmt : -1;
+  return group == 128 ? kFmtW4A16 : group == 64 ? kFmtW4G64 : group == 32 ? kFmtW4G32 : -1;
+}
+
+// Whether the operands lie as the prefill GEMM's loads take them: rows and
+// codes by 16 bytes, scales by dwords.
+bool tile_aligned(std::initializer_list<const void*> rows_and_codes,
+                  std::initializer_list<const void*> scales) {
+  uintptr_t any = 0, sc = 0;
+  for (const void* p : rows_and_codes) any |= reinterpret_cast<uintptr_t>(p);
+  for (const void* p : scales) sc |= reinterpret_cast<uintptr_t>(p);
+  return (any & 15) == 0 && (sc & 3) == 0;
+}
+
+// Whether the prefill GEMM (tile_gemm.hip) takes a dense launch: whole 128-wide
+// k-steps, 32-bit byte offsets, paired rows (W4A16) and operands aligned for
+// its loads (what the kernels it stands in for read in 2- and 4-byte pieces
+// may lie anywhere).
+bool tile_fits(const GemmArgs& g, int fmt) {
+  const int tf = tile_format(fmt, g.group);
+  if (tf < 0 || g.k % 128 != 0 || g.a_rows <= 0) return false;
+  if (g.a_rows * g.k * 2 > kMaxDirectBytes || g.n * g.k > kMaxDirectBytes) return false;
+  if (fmt_is_w4(tf) && !(g.a_pair && g.a_neg)) return false;
+  return tile_aligned({fmt_is_w4(tf) ? g.a_pair : g.a, g.wp[0], g.wp[1], g.wp[2], g.out[0],
+                       g.out[1], g.out[2]},
+                      {g.ws[0], g.ws[1], g.ws[2]});
+}
 
 // Dense products (dense GEMM, fused QKV, MXFP4 GEMM) from 16 rows: the
 // streaming kernel with 64-row tiles (weights in a register ring, activations
@@ -3142,6 +2776,8 @@ bool wide_cols_for(int64_t tiles, int64_t n) { return tiles * ((n + 63) / 64) >=
 template <int FMT>
 int dense_launch(const GemmArgs& g, int64_t tiles, hipStream_t s, const char* what) {
   const bool lds = path_choice(kKnobDenseGemm) == 1;
+  if (!lds && tile_fits(g, FMT))
+    return tile_gemm_launch(tile_format(FMT, g.group), 1, g, Mode::Dense, tiles, s, what);
   if (!lds && stream_fits(g.k, 4, g.group, FMT != kFmtW4A16))
     return stream_launch<FMT, 1>(g, Mode::Dense, tiles, 4, s, what);
   return gemm_launch<FMT, 1>(g, Mode::Dense, tiles, wide_cols_for(tiles * g.outputs, g.n), s, what);
@@ -3233,28 +2869,52 @@ void dense_args(GemmArgs& g, const uint16_t* x, int64_t m, int64_t n, int64_t k,
   g.act = kActSwiglu;
 }
 
-// Workspace of a dense W4A16 product whose 64-row launches load their rows
-// directly: the rows paired in the weight decode's k order and their group
-// sums (G = 128, k % 128 == 0, from 16 rows); 0 where that form does not apply.
+// Group sums of one paired row (pair_rows_kernel): a float per 128-wide k-step
+// at G = 128, four at G = 32 and 64.
+int64_t pair_sums(int64_t k, int64_t group) { return (k / 128) * (group == 128 ? 1 : 4); }
+
+// Workspace of a dense W4A16 product on the prefill GEMM, which loads its
+// rows directly: the rows paired in the weight decode's k order and their
+// group sums (G <= 128, k % 128 == 0, from 16 rows); 0 where it does not apply.
 int64_t dense_pair_bytes(int64_t m, int64_t k, int64_t group) {
-  if (m < 16 || group != 128 || k % 128 != 0) return 0;
+  if (m < 16 || (group != 32 && group != 64 && group != 128) || k % 128 != 0) return 0;
   return static_cast<int64_t>(align_up(static_cast<size_t>(m * k * 2)) +
-                              align_up(static_cast<size_t>(m * (k / 128) * 4)));
+                              align_up(static_cast<size_t>(m * pair_sums(k, group) * 4)));
+}
+
+// Workspace of a dense product on the prefill GEMM: the paired rows (W4A16),
+// then the sums of a product split over k where that pays.
+int64_t dense_ws_bytes(bool mx, int64_t m, int64_t n, int64_t k, int64_t group, int64_t outputs) {
+  const int64_t pairs = mx ? 0 : dense_pair_bytes(m, k, group);
+  if (k % 128 != 0 || m < 1 || (!mx && pairs == 0)) return pairs;
+  return pairs + tile_gemm_split_bytes(mx, m, n, k, outputs);
+}
+
+// Points the launch at the split sums when the workspace holds them (a
+// workspace without that room runs the product unsplit).
+void dense_split(GemmArgs& g, bool mx, int64_t group, void* workspace, int64_t workspace_bytes) {
+  const int64_t pairs = mx ? 0 : dense_pair_bytes(g.dense_rows, g.k, group);
+  const int64_t need = dense_ws_bytes(mx, g.dense_rows, g.n, g.k, group, g.outputs);
+  if (workspace != nullptr && need > pairs && workspace_bytes >= need &&
+      (reinterpret_cast<uintptr_t>(workspace) & 15) == 0)
+    g.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + pairs);
 }
 
 // The pre-pass of the direct form: pairs x into the workspace and points the
-// launch at it.
+// launch at it. At G = 32 and 64 a call without the workspace keeps the
+// staged form, which needs none.
 int dense_pairs(GemmArgs& g, const uint16_t* x, int64_t m, int64_t k, int64_t group,
                 void* workspace, int64_t workspace_bytes, hipStream_t s, const char* what) {
   const int64_t need = dense_pair_bytes(m, k, group);
   if (need == 0) return LK_OK;
-  LK_REQUIRE(workspace != nullptr && workspace_bytes >= need,
-             "%s: workspace too small: %lld < %lld bytes", what, (long long)workspace_bytes,
+  const bool have = workspace != nullptr && workspace_bytes >= need;
+  if (!have && group != 128) return LK_OK;
+  LK_REQUIRE(have, "%s: workspace too small: %lld < %lld bytes", what, (long long)workspace_bytes,
              (long long)need);
   auto* xp = static_cast<uint16_t*>(workspace);
   auto* neg = reinterpret_cast<float*>(static_cast<char*>(workspace) +
                                        align_up(static_cast<size_t>(m * k * 2)));
-  if (int rc = pair_rows_launch(x, xp, neg, m, k, s)) return rc;
+  if (int rc = pair_rows_launch(x, xp, neg, m, k, group, s)) return rc;
   g.a_pair = xp;
   g.a_neg = neg;
   g.a_rows = m;
@@ -3431,8 +3091,20 @@ int lk_w4a16_dense_gemm(const uint16_t* x, const uint8_t* packed, const uint16_t
   return dense_launch<kFmtW4A16>(g, tiles, as_stream(stream), "lk_w4a16_dense_gemm");
 }
 
+int64_t lk_dense_gemm_workspace(int64_t m, int64_t n, int64_t k, int64_t group_size,
+                                int64_t outputs, int mxfp4) {
+  if (m < 0 || n <= 0 || k <= 0 || group_size <= 0 || outputs < 1 || outputs > 3) return -1;
+  return dense_ws_bytes(mxfp4 != 0, m, n, k, group_size, outputs);
+}
+
 int lk_mxfp4_gemm(const uint16_t* x, const uint8_t* packed, const uint8_t* scale, uint16_t* y,
                   int64_t m, int64_t n, int64_t k, int act_f16, void* stream) {
+  return lk_mxfp4_gemm_ws(x, packed, scale, y, m, n, k, act_f16, nullptr, 0, stream);
+}
+
+int lk_mxfp4_gemm_ws(const uint16_t* x, const uint8_t* packed, const uint8_t* scale, uint16_t* y,
+                     int64_t m, int64_t n, int64_t k, int act_f16, void* workspace,
+                     int64_t workspace_bytes, void* stream) {
   LK_REQUIRE(packed && scale && y, "null pointer argument");
   LK_REQUIRE(m >= 0 && n > 0, "reduction and output dimensions must be nonzero");
   if (int rc = check_format(true, k, 32)) return rc;
@@ -3441,10 +3113,11 @@ int lk_mxfp4_gemm(const uint16_t* x, const uint8_t* packed, const uint8_t* scale
   LK_REQUIRE(m < (1LL << 30), "too many rows");
   GemmArgs g{};
   dense_args(g, x, m, n, k, 32);
-  g.a_rows = m;  // bf16 rows load directly (the fp16 form stages them)
+  g.a_rows = m;  // rows load directly
   g.wp[0] = g.wp[1] = g.wp[2] = packed;
   g.ws[0] = g.ws[1] = g.ws[2] = scale;
   g.out[0] = g.out[1] = g.out[2] = y;
+  dense_split(g, true, 32, workspace, workspace_bytes);
   const int64_t tiles = (m + kTileRows - 1) / kTileRows;
   if (act_f16)
     return dense_launch<kFmtMxF16>(g, tiles, as_stream(stream), "lk_mxfp4_gemm");
@@ -3528,7 +3201,7 @@ int lk_w4a16_fused_qkv(const uint16_t* x, const uint8_t* q_packed, const uint16_
 
 int64_t lk_w4a16_dense_gemm_workspace(int64_t m, int64_t k, int64_t group_size) {
   if (m < 0 || k <= 0 || group_size <= 0) return -1;
-  return dense_pair_bytes(m, k, group_size);
+  return group_size == 128 ? dense_pair_bytes(m, k, group_size) : 0;
 }
 
 int lk_w4a16_dense_gemm_ws(const uint16_t* x, const uint8_t* packed, const uint16_t* scales,
@@ -3550,6 +3223,7 @@ int lk_w4a16_dense_gemm_ws(const uint16_t* x, const uint8_t* packed, const uint1
   if (int rc = dense_pairs(g, x, m, k, group_size, workspace, workspace_bytes, s,
                            "lk_w4a16_dense_gemm_ws"))
     return rc;
+  dense_split(g, false, group_size, workspace, workspace_bytes);
   const int64_t tiles = (m + kTileRows - 1) / kTileRows;
   return dense_launch<kFmtW4A16>(g, tiles, s, "lk_w4a16_dense_gemm_ws");
 }
@@ -3588,6 +3262,7 @@ int lk_w4a16_fused_qkv_ws(const uint16_t* x, const uint8_t* q_packed, const uint
   if (int rc = dense_pairs(g, x, m, k, group_size, workspace, workspace_bytes, s,
                            "lk_w4a16_fused_qkv_ws"))
     return rc;
+  dense_split(g, false, group_size, workspace, workspace_bytes);
   const int64_t tiles = (m + kTileRows - 1) / kTileRows;
   return dense_launch<kFmtW4A16>(g, tiles, s, "lk_w4a16_fused_qkv_ws");
 }
@@ -3671,8 +3346,16 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
   // 64-row tiles load activations directly (32-bit byte offsets)
   if (mt == 4 && (tokens * h * 2 > kMaxDirectBytes || entries * i * 2 > kMaxDirectBytes)) mt = 0;
   const int tr = mt == 1 ? kSmallTileRows : kTileRows;
-  // W4A16 G = 128 on 64-row tiles: x and the activations go in paired
-  const bool paired = !mx && mt == 4 && group == 128;
+  // MXFP4 on the scaled fp4 MFMA: x and the activations go in as fp8 hi + lo
+  const bool f8 = mx && mt != 0 && h % 128 == 0 && i % 128 == 0 && mxfp4_scaled_mfma();
+  // 64-row tiles: the prefill GEMM where it takes both products
+  const int fmt = mx ? kFmtMxBf16 : kFmtW4A16;
+  const bool tile = mt == 4 && !f8 && tile_format(fmt, group) >= 0 && h % 128 == 0 && i % 128 == 0 &&
+                    i * h <= kMaxDirectBytes &&
+                    tile_aligned({x, w1_packed, w3_packed, w2_packed},
+                                 {w1_scales, w3_scales, w2_scales});
+  // W4A16 on 64-row tiles: x and the activations go in paired
+  const bool paired = !mx && tile;
   // ...and when the batch takes the router launch (the 64-row tiles route
   // neither in the GEMM nor in the one-launch schedule), that launch also
   // pairs them (route_pair_kernel): one launch instead of two; the path knob
@@ -3686,8 +3369,6 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
   // the down GEMM and the combine kernel; it reads an expert's W2 once per
   // route that uses it rather than once per call.
   const bool w2_rows = !mx && tokens <= kW2RowsMaxTokens && w2_rows_fits(routes, i);
-  // MXFP4 on the scaled fp4 MFMA: x and the activations go in as fp8 hi + lo
-  const bool f8 = mx && mt != 0 && h % 128 == 0 && i % 128 == 0 && mxfp4_scaled_mfma();
   SplitBufs xs{}, as{};
   if (f8) {
     xs = split_bufs(ws + l.x_split, tokens * h);
@@ -3699,8 +3380,6 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
   g.perm = perm;
   g.tiles = tiles;
   g.tile_count = count;
-  g.mtiles = mtiles;
-  g.mtile_count = mcount;
   g.group = group;
   g.routes = routes;
   g.outputs = 1;
@@ -3716,7 +3395,7 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
     g.a_neg = reinterpret_cast<float*>(ws + l.x_neg);
     if (!route_pairs) {
       if (int rc = pair_rows_launch(x, const_cast<uint16_t*>(g.a_pair),
-                                    const_cast<float*>(g.a_neg), tokens, h, s))
+                                    const_cast<float*>(g.a_neg), tokens, h, group, s))
         return rc;
     }
   }
@@ -3732,6 +3411,10 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
   g.k = h;
   g.wstride = i * h / 2;
   g.sstride = i * (h / group);
+  if (tile) {  // the merged list: an expert's short last tile joins the one before it
+    g.tiles = mtiles;
+    g.tile_count = mcount;
+  }
   const Mode gu_mode = w2_rows ? Mode::GatherScatter : Mode::Gather;
   // down projection: sorted activation rows, outputs scattered to (token, route) rows
   auto down_args = [&](GemmArgs d) {
@@ -3841,7 +3524,7 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
                      ? route_pair_launch(logits, bias, expert_indices, weights, tokens, experts - 1,
                                          top_k, routed_scaling_factor, renormalize, x,
                                          const_cast<uint16_t*>(g.a_pair),
-                                         const_cast<float*>(g.a_neg), h, s)
+                                         const_cast<float*>(g.a_neg), h, group, s)
                      : lk_moe_router(logits, bias, expert_indices, weights, tokens, experts - 1,
                                      top_k, routed_scaling_factor, renormalize, stream))
       return rc;
@@ -3856,6 +3539,8 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
                : f8 ? stream_launch<kFmtMxF8, 2>(g, Mode::Gather, tb, mt, s, "moe gate/up gemm")
                : split ? persist_fmt<1>(mx, g, Mode::Gather, tb, s, "moe gate/up gemm",
                                         PsForm::SplitGateUp, true)
+               : tile  ? tile_gemm_launch(tile_format(fmt, group), 2, g, Mode::Gather, tb, s,
+                                          "moe gate/up gemm")
                : mt    ? stream_fmt<2>(mx, g, gu_mode, tb, mt, s, "moe gate/up gemm")
                        : launch_fmt<2>(mx, g, gu_mode, tb, wide_cols_for(tb, i), s,
                                        "moe gate/up gemm"))
@@ -3871,6 +3556,8 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
   if (int rc = f8 ? stream_launch<kFmtMxF8, 1>(g, Mode::Scatter, tb, mt, s, "moe down gemm")
                : split ? persist_fmt<1>(mx, g, Mode::Scatter, tb, s, "moe down gemm",
                                         PsForm::SwiDown, true)
+               : tile  ? tile_gemm_launch(tile_format(fmt, group), 1, g, Mode::Scatter, tb, s,
+                                          "moe down gemm")
                : mt    ? stream_fmt<1>(mx, g, Mode::Scatter, tb, mt, s, "moe down gemm")
                        : launch_fmt<1>(mx, g, Mode::Scatter, tb, wide_cols_for(tb, h), s,
                                        "moe down gemm"))

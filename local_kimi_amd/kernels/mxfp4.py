@@ -62,16 +62,21 @@ def _gemm(entry: str, activations, weight_packed, weight_scale) -> torch.Tensor:
     if m == 0:
         return out
     x, p, s = _w._c(activations), _w._c(weight_packed), _w._c(weight_scale)
+    args = [x.data_ptr(), p.data_ptr(), s.data_ptr(), out.data_ptr(), m, n, k,
+            int(activations.dtype == torch.float16)]
+    if entry == "lk_mxfp4_gemm_ws":  # room for the sums of a product split over k
+        ws = _w.workspace(_lib.query("lk_dense_gemm_workspace", m, n, k, MXFP4_GROUP_SIZE, 1, 1),
+                          activations.device)
+        args += [ws.data_ptr(), ws.numel()]
     with torch.cuda.device(activations.device):
-        _lib.call(entry, x.data_ptr(), p.data_ptr(), s.data_ptr(), out.data_ptr(), m, n, k,
-                  int(activations.dtype == torch.float16), _w._stream(activations.device))
+        _lib.call(entry, *args, _w._stream(activations.device))
     return out
 
 
 def mxfp4_gemm(activations: torch.Tensor, weight_packed: torch.Tensor,
                weight_scale: torch.Tensor) -> torch.Tensor:
     """``activations @ dequant(weight).T`` without a decoded weight tensor."""
-    return _gemm("lk_mxfp4_gemm", activations, weight_packed, weight_scale)
+    return _gemm("lk_mxfp4_gemm_ws", activations, weight_packed, weight_scale)
 
 
 def mxfp4_linear(activations, weight_packed, weight_scale) -> torch.Tensor:

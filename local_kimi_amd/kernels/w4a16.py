@@ -106,13 +106,13 @@ def _dense(entry: str, activations, packed_weights, scales):
 
 
 def _dense_gemm(activations, packed_weights, scales):
-    """The MFMA GEMM with its direct-load workspace (the paired rows and their
-    group sums, G = 128) from the torch caching allocator."""
+    """The MFMA GEMM with its workspace (the paired rows with their group sums,
+    and the sums of a product split over k) from the torch caching allocator."""
     m, n, k, g = _validate_dense(activations, packed_weights, scales)
     out = torch.empty((m, n), dtype=torch.bfloat16, device=activations.device)
     if m == 0:
         return out
-    ws = workspace(_lib.query("lk_w4a16_dense_gemm_workspace", m, k, g), activations.device)
+    ws = workspace(_lib.query("lk_dense_gemm_workspace", m, n, k, g, 1, 0), activations.device)
     x, p, s = _c(activations), _c(packed_weights), _c(scales)
     with torch.cuda.device(activations.device):
         _lib.call("lk_w4a16_dense_gemm_ws", x.data_ptr(), p.data_ptr(), s.data_ptr(),
@@ -425,7 +425,7 @@ def fused_qkv_w4a16(activations, q_packed, q_scales, k_packed, k_scales, v_packe
         return tuple(outs)
     x = _c(activations)
     w = [_c(t) for t in (q_packed, q_scales, k_packed, k_scales, v_packed, v_scales)]
-    ws = workspace(_lib.query("lk_w4a16_dense_gemm_workspace", m, k, g), dev)
+    ws = workspace(_lib.query("lk_dense_gemm_workspace", m, n, k, g, 3, 0), dev)
     with torch.cuda.device(dev):
         _lib.call("lk_w4a16_fused_qkv_ws", x.data_ptr(), *(t.data_ptr() for t in w),
                   *(o.data_ptr() for o in outs), m, n, k, g, ws.data_ptr(), ws.numel(),
