@@ -22,8 +22,9 @@
 //   y += s_g * (sum_{k in g} x * (q + 136) - 136 * sum_{k in g} x).
 // The positions of one MFMA must share a group: with G >= 128 a lane's 16
 // contiguous packed bytes (32 codes) feed the 4 MFMAs of one 128-wide k-step;
-// with G = 32 or 64 each MFMA covers 32 consecutive codes and a lane loads
-// one dword per MFMA.
+// with G = 32 or 64 each MFMA covers 32 consecutive codes: the lane blocks
+// swap the dwords of 16-byte loads (transpose4), or a lane loads one dword per
+// MFMA where the shape or the alignment rules those out.
 
 #include <stdlib.h>
 #include <string.h>
@@ -1378,13 +1379,32 @@ __device__ inline void ps_stage_store(uint4* afrag, float* offs, int frag, int c
 // are issued back to back (they are the two halves of one 128-byte line of
 // the weight row, so the line is fetched once: requested apart, each half
 // costs a fetch of its own), and one scale load serves both steps (W4A16
-// G = 128: the bf16 pair, low half = step 2q; G = 64 and 32: four and eight
-// bf16; MXFP4: eight E8M0 bytes, four per step). Whole-dword scale loads keep the ring free of narrow loads, whose
+// G = 128: the bf16 pair, low half = step 2q; G = 64 and 32: the pair's two
+// and four dwords of bf16, one per lane block, spread by ps_scale_dwords where
+// they are used: held whole they are up to 12 registers of ring more, which
+// spilled; MXFP4: eight E8M0 bytes, four per step). Whole-dword scale loads keep the ring free of narrow loads, whose
 // zero-extension the compiler otherwise places at the loop latch, where it
 // waits for every load in flight.
+// Step h's scale dwords (G = 32: dwords 2 h and 2 h + 1 of the pair's four, in
+// lane blocks 0 .. 3; G = 64: dword h of two, in lane blocks 0, 1, 0, 1) in
+// every lane.
+template <int CHAIN>
+__device__ inline void ps_scale_dwords(uint32_t s, int h, uint32_t (&d)[CHAIN == 1 ? 2 : 1]) {
+  if constexpr (CHAIN == 1) {
+    const auto half = __builtin_amdgcn_permlane32_swap(s, s, false, false);
+    const uint32_t two = half[h];  // lane blocks 2 h, 2 h + 1, 2 h, 2 h + 1
+    const auto row = __builtin_amdgcn_permlane16_swap(two, two, false, false);
+    d[0] = row[0];
+    d[1] = row[1];
+  } else {
+    const auto row = __builtin_amdgcn_permlane16_swap(s, s, false, false);
+    d[0] = row[h];
+  }
+}
+
 template <int FMT, int MATS, int NT>
 struct PsPair {
-  static constexpr int kSw = fmt_is_w4(FMT) ? 4 / fmt_chain(FMT) : 2;  // scale dwords per pair
+  static constexpr int kSw = fmt_is_w4(FMT) ? 1 : 2;  // scale dwords per lane and pair
   uint32_t w[2][MATS][NT][4];
   uint32_t s[MATS][NT][kSw];
 
@@ -1398,18 +1418,13 @@ struct PsPair {
       for (int nt = 0; nt < NT; ++nt) {
         const void* sp;
         if constexpr (fmt_is_w4(FMT))
-          sp = static_cast<const uint16_t*>(srow[mi][nt]) + step0 * (4 / fmt_chain(FMT));
+          sp = static_cast<const uint16_t*>(srow[mi][nt]) + step0 * (4 / fmt_chain(FMT)) +
+               2 * (jq & (4 / fmt_chain(FMT) - 1));
         else
           sp = static_cast<const uint8_t*>(srow[mi][nt]) + static_cast<int64_t>(step0) * 4;
         if (!live) sp = dummy;
         if constexpr (kSw == 1) {
           s[mi][nt][0] = *static_cast<const uint32_t*>(sp);
-        } else if constexpr (kSw == 4) {
-          const uint4 v = *static_cast<const uint4*>(sp);
-          s[mi][nt][0] = v.x;
-          s[mi][nt][1] = v.y;
-          s[mi][nt][2] = v.z;
-          s[mi][nt][3] = v.w;
         } else {
           const uint2 v = *static_cast<const uint2*>(sp);
           s[mi][nt][0] = v.x;
@@ -1939,14 +1954,12 @@ w4a16_persist_kernel(const GemmArgs g, int nbuf) {
       for (int mi = 0; mi < MATS; ++mi)
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
+          uint32_t sd[kChain == 1 ? 2 : 1];
+          ps_scale_dwords<kChain>(wj.s[mi][nt][0], h, sd);
 #pragma unroll
-          for (int q = 0; q < kGroups4; ++q) {  // decoded as below
-            const int e = h * kGroups4 + q;
-            if (e & 1)
-              asm("v_and_b32 %0, 0xffff0000, %1" : "=v"(sc[mi][nt][q]) : "v"(wj.s[mi][nt][e >> 1]));
-            else
-              asm("v_lshlrev_b32 %0, 16, %1" : "=v"(sc[mi][nt][q]) : "v"(wj.s[mi][nt][e >> 1]));
-          }
+          for (int q = 0; q < kGroups4; ++q)
+            sc[mi][nt][q] = __uint_as_float((q & 1) ? (sd[q >> 1] & 0xFFFF0000u)
+                                                    : (sd[q >> 1] << 16));
 #pragma unroll
           for (int t = 0; t < 4; ++t) wt[mi][nt][t] = wj.w[h][mi][nt][t];
           transpose4(wt[mi][nt]);
@@ -2767,11 +2780,11 @@ bool tile_fits(const GemmArgs& g, int fmt) {
                       {g.ws[0], g.ws[1], g.ws[2]});
 }
 
-// Dense products (dense GEMM, fused QKV, MXFP4 GEMM) from 16 rows: the
-// streaming kernel with 64-row tiles (weights in a register ring, activations
-// in LDS passes) where it covers the format, else the LDS-staged GEMM. On the
-// fused QKV projection of 2048 tokens ([2048, 2304] x [2304, 3 x 4096]) the
-// streaming kernel takes 226 us, the LDS-staged GEMM 421 us. The path knob
+// Dense products (dense GEMM, fused QKV, MXFP4 GEMM) from 16 rows: the prefill
+// GEMM where it takes the operands (2048 x 2304 x 3 x 4096 at G = 128: 123 us
+// against 156 on the streaming kernel, 421 on the LDS-staged GEMM), else the
+// streaming kernel with 64-row tiles (k not a multiple of 128, operands off
+// its alignments), else the LDS-staged GEMM (wider groups). The path knob
 // dense_gemm=lds forces the LDS-staged GEMM.
 template <int FMT>
 int dense_launch(const GemmArgs& g, int64_t tiles, hipStream_t s, const char* what) {
@@ -3368,7 +3381,7 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
   // token-major launch does W2, the combine and the shared expert, instead of
   // the down GEMM and the combine kernel; it reads an expert's W2 once per
   // route that uses it rather than once per call.
-  const bool w2_rows = !mx && tokens <= kW2RowsMaxTokens && w2_rows_fits(routes, i);
+  bool w2_rows = !mx && tokens <= kW2RowsMaxTokens && w2_rows_fits(routes, i);
   SplitBufs xs{}, as{};
   if (f8) {
     xs = split_bufs(ws + l.x_split, tokens * h);
@@ -3415,7 +3428,6 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
     g.tiles = mtiles;
     g.tile_count = mcount;
   }
-  const Mode gu_mode = w2_rows ? Mode::GatherScatter : Mode::Gather;
   // down projection: sorted activation rows, outputs scattered to (token, route) rows
   auto down_args = [&](GemmArgs d) {
     d.a = act;
@@ -3446,11 +3458,17 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
   // against 81.4 us fused, at 16 tokens 34.8 against 38.1 us: units of half
   // the bytes shorten the launch's tail, where each block's last units
   // stream alone.
-  const bool split =
-      mt == 1 && !f8 && !w2_rows && moe_act_mult(entries) == 2 &&
+  const bool split_fits =
+      mt == 1 && !f8 && moe_act_mult(entries) == 2 &&
       path_choice(kKnobMoeSplitSwiglu) != 1 &&
       persist_fmt<1>(mx, g, Mode::Gather, tb, s, "", PsForm::SplitGateUp, false) == 0 &&
       persist_fmt<1>(mx, down_args(g), Mode::Scatter, tb, s, "", PsForm::SwiDown, false) == 0;
+  // G = 32 at widths of the persistent kernels: their two-matrix gate/up unit,
+  // which the token-major W2 follows, does not fit the registers (4 tokens of
+  // the Kimi-Linear layer 73 us with it, 41 with the split form)
+  if (group == 32 && h % 256 == 0 && i % 256 == 0) w2_rows = false;
+  const bool split = split_fits && !w2_rows;
+  const Mode gu_mode = w2_rows ? Mode::GatherScatter : Mode::Gather;
   // Batches of at most 8 tokens (one per wave) on the persistent 16-row
   // GEMMs: the gate/up GEMM routes and schedules the batch in every block
   // (route_schedule_block) where that launch applies, with no router or
