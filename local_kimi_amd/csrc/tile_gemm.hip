@@ -420,14 +420,25 @@ __global__ void __launch_bounds__(W * kWave, TILES == 4 ? 2 : 3) tile_gemm_kerne
     tile = j / band;
     cb_all = (id & 7) * band + (j - tile * band);
   } else {
-    // schedule modes: XCD x walks the x-th eighth of the list, a tile's column
-    // blocks together, so tiles of one expert meet in one L2
+    // XCD x takes an eighth of the list, a tile's column blocks together.
+    // Schedule modes: whole tiles, consecutive ones, so tiles of one expert
+    // meet in one L2 (an even split of the blocks measured 403 against 381 us
+    // on the block of 777 tokens). Dense: an even split of the blocks (whole
+    // tiles left XCDs idle where the tiles are few: 468 blocks 65 against 44 us).
     const int count = DENSE ? (g.dense_rows + kTileRows - 1) / kTileRows : *g.tile_count;
-    const int chunk = (count + 7) >> 3;
     const int j = id >> 3;
-    if (j >= chunk * per_tile) return;
-    tile = (id & 7) * chunk + j / per_tile;
-    cb_all = j % per_tile;
+    if constexpr (DENSE) {
+      const int units = count * per_tile, share = (units + 7) >> 3;
+      const int unit = (id & 7) * share + j;
+      if (j >= share || unit >= units) return;
+      tile = unit / per_tile;
+      cb_all = unit - tile * per_tile;
+    } else {
+      const int chunk = (count + 7) >> 3;
+      if (j >= chunk * per_tile) return;
+      tile = (id & 7) * chunk + j / per_tile;
+      cb_all = j % per_tile;
+    }
   }
   const int osel = cb_all / g.col_blocks;
   const int cb = cb_all - osel * g.col_blocks;
@@ -546,19 +557,25 @@ int launch_fmt(int fmt, const GemmArgs& g, Mode mode, dim3 blocks, hipStream_t s
 
 namespace {
 
-// Column blocks and k-split of a dense product of m rows: 128 columns a block
-// where 256 leave slots idle (two 256-column blocks fit a CU, three 128-column
-// ones; 333 x 2304 x 9216 MXFP4: 19.4 against 38.4 us, 2048 x 2304 x 12288:
-// 143 against 126), and k in runs of at least kTgRunSteps k-steps where even
-// those leave CUs idle. Estimated microseconds, fitted to measurements at 16
+// Column blocks and k-split of a dense product of m rows. 256-column blocks
+// where they fill their rounds of 512 (two fit a CU), else 128-column ones
+// (three fit a CU, and their partial rounds cost less): r = blocks / 512,
+// 256 against 128 columns in us: r = 0.7 40.9 : 38.9, 0.91 44.3 : 49.5, 1.13
+// 64.5 : 56.7, 1.5 65 : 69, 1.97 80.6 : 87, 2.25 101.9 : 100.2, 3 118 : 129
+// (k = 2304, G = 128); 333 x 2304 x 9216 MXFP4 (0.42) 25.3 : 19.4.
+// K goes in runs of at least kTgRunSteps k-steps where even 128-column blocks
+// leave CUs idle. Estimated microseconds, fitted to measurements at 16
 // to 1500 rows: a k-step of one block alone on its CU takes 0.65 + 0.17 a
 // 16-row subtile (MXFP4: 0.35 + 0.1), 0.6 of that more for each further block
 // on the CU; runs cost the reduce launch (5, with its launch on the host) and
 // their fp32 sums written and read at 6 TB/s; a split has to gain kTgGain.
 // 64 x 9216 -> 2304 at G = 32: 32 us in 8 runs against 70; 1000 rows 97
 // against 126; 200 x 2304 -> 9216 stays whole (31.4 against 34.2).
-constexpr int64_t kTgWideBlocks = 512;
+constexpr double kTgWideSlots = 512.0;
 constexpr int64_t kTgRunSteps = 4;
+// shorter products stay whole (little to gain, and their outputs stay the
+// bits of the kernels without a workspace)
+constexpr int64_t kTgSplitSteps = 24;
 constexpr int64_t kTgMaxRuns = 16;
 constexpr double kTgGain = 6.0;
 
@@ -569,8 +586,11 @@ struct DensePlan {
 
 DensePlan dense_plan(bool mx, int64_t m, int64_t n, int64_t k, int64_t outputs, bool may_split) {
   const int64_t tiles = (m + kTileRows - 1) / kTileRows, ksteps = k / 128;
-  DensePlan p{tiles * ((n + 255) / 256) * outputs < kTgWideBlocks, ksteps, 1};
-  if (!p.narrow || !may_split) return p;
+  const double r = static_cast<double>(tiles * ((n + 255) / 256) * outputs) / kTgWideSlots;
+  const double part = r - static_cast<double>(static_cast<int64_t>(r));
+  const bool wide = r >= 3.0 || (r >= 0.8 && (part == 0.0 || part >= 0.4));
+  DensePlan p{!wide, ksteps, 1};
+  if (!p.narrow || !may_split || ksteps < kTgSplitSteps) return p;
   const double blocks = static_cast<double>(tiles * ((n + 127) / 128) * outputs);
   const double subtiles = static_cast<double>((std::min<int64_t>(m, kTileRows) + 15) / 16);
   const double step = mx ? 0.35 + 0.1 * subtiles : 0.65 + 0.17 * subtiles;
