@@ -84,7 +84,7 @@ def kda_decode_step(state: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: to
     work = _dense(state)
     qc, kc, vc, dc, bc = (_w._c(t) for t in (q, k, v, decay, beta))
     out = torch.empty((batch, heads, d_v), dtype=torch.float32, device=state.device)
-    with torch.cuda.device(state.device):
+    with _w._on(state.device):
         _lib.call("lk_kda_decode_step", work.data_ptr(), qc.data_ptr(), kc.data_ptr(),
                   vc.data_ptr(), dc.data_ptr(), bc.data_ptr(), out.data_ptr(), batch, heads,
                   d_k, d_v, float(scale), _w._stream(state.device))
@@ -163,7 +163,7 @@ def fused_short_conv_triple(q_in: torch.Tensor, k_in: torch.Tensor, v_in: torch.
     work = [s if s.is_contiguous() else s.contiguous() for s in states]
     outs = [torch.empty((batch, 1, channels), dtype=q_in.dtype, device=q_in.device)
             for _ in range(3)]
-    with torch.cuda.device(q_in.device):
+    with _w._on(q_in.device):
         _lib.call("lk_kda_short_conv_triple", *(t.data_ptr() for t in ins),
                   *(t.data_ptr() for t in work), *(t.data_ptr() for t in weights),
                   *(t.data_ptr() for t in outs), batch, channels, vcode, wcode,
@@ -239,7 +239,7 @@ def fused_kda_gates(raw_decay: torch.Tensor, dt_bias: torch.Tensor, a_log: torch
     beta = torch.empty(tuple(raw_beta.shape), dtype=torch.float32, device=dev)
     q_out = torch.empty((batch, sequence, num_heads, head_dim), dtype=torch.float32, device=dev)
     k_out = torch.empty_like(q_out)
-    with torch.cuda.device(dev):
+    with _w._on(dev):
         _lib.call("lk_kda_gates", raw_decay.data_ptr(), bias.data_ptr(), rate.data_ptr(),
                   raw_beta.data_ptr(), q.data_ptr(), k.data_ptr(), decay.data_ptr(),
                   beta.data_ptr(), q_out.data_ptr(), k_out.data_ptr(), batch * sequence,
@@ -310,7 +310,7 @@ def kda_decode_layer(q_in: torch.Tensor, k_in: torch.Tensor, v_in: torch.Tensor,
     rate = a_log.float().reshape(num_heads).contiguous()
     out = torch.empty((batch, num_heads, head_dim), dtype=torch.float32, device=state.device)
     s = head_dim ** -0.5 if scale is None else float(scale)
-    with torch.cuda.device(state.device):
+    with _w._on(state.device):
         _lib.call("lk_kda_decode_layer", *(t.data_ptr() for t in ins),
                   *(t.data_ptr() for t in conv_work), *(t.data_ptr() for t in weights),
                   raw_decay.data_ptr(), bias.data_ptr(), rate.data_ptr(), raw_beta.data_ptr(),
@@ -346,7 +346,7 @@ def _layer_split(ins, states, outs, weights, raw_decay, dt_bias, a_log, raw_beta
     rate = a_log.float().reshape(num_heads).contiguous()
     out = torch.empty((batch, num_heads, head_dim), dtype=torch.float32, device=state.device)
     s = head_dim ** -0.5 if scale is None else float(scale)
-    with torch.cuda.device(state.device):
+    with _w._on(state.device):
         _lib.call("lk_kda_decode_layer_split", *(t.data_ptr() for t in ins),
                   *(t.data_ptr() for t in src), *(t.data_ptr() for t in outs),
                   *(t.data_ptr() for t in weights), raw_decay.data_ptr(), bias.data_ptr(),

@@ -57,7 +57,7 @@ def moe_schedule(expert_indices: torch.Tensor, experts: int, shared_expert: int 
     count = torch.empty((1,), dtype=torch.int32, device=dev)
     ws = _w.workspace(ws_bytes, dev)
     idx = _w._c(expert_indices)
-    with torch.cuda.device(dev):
+    with _w._on(dev):
         _lib.call("lk_moe_schedule", idx.data_ptr(), tokens, routes, experts, shared_expert,
                   tile_rows, offsets.data_ptr(), perm.data_ptr(), tiles.data_ptr(), count.data_ptr(),
                   ws.data_ptr(), ws.numel(), _w._stream(dev))
@@ -116,7 +116,7 @@ def moe_router(logits: torch.Tensor, bias: torch.Tensor | None, top_k: int, *,
         return idx, w
     lg = _w._c(logits)
     b = _w._c(bias) if bias is not None else None
-    with torch.cuda.device(logits.device):
+    with _w._on(logits.device):
         if num_expert_group > 1:
             _lib.call("lk_moe_router_grouped", lg.data_ptr(),
                       b.data_ptr() if b is not None else None, idx.data_ptr(), w.data_ptr(),
@@ -162,7 +162,7 @@ def router_logits(hidden: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     if weight.dtype == torch.float16:
         weight = weight.float()
     x, w = _w._c(hidden), _w._c(weight)
-    with torch.cuda.device(hidden.device):
+    with _w._on(hidden.device):
         _lib.call("lk_router_logits", x.data_ptr(), w.data_ptr(), out.data_ptr(), tokens, experts, h,
                   int(w.dtype == torch.float32), _w._stream(hidden.device))
     return out
@@ -302,7 +302,7 @@ def w4a16_moe_forward(hidden: torch.Tensor, logits: torch.Tensor, bias: torch.Te
     x, lg = c(hidden), c(logits)
     b = c(bias) if bias is not None else None
     args = [c(t) for t in (w1_packed, w1_scales, w3_packed, w3_scales, w2_packed, w2_scales)]
-    with torch.cuda.device(dev):
+    with _w._on(dev):
         _lib.call("lk_w4a16_moe_forward", x.data_ptr(), lg.data_ptr(),
                   b.data_ptr() if b is not None else None, *(t.data_ptr() for t in args),
                   y.data_ptr(), idx.data_ptr(), w.data_ptr(), ws.data_ptr(), ws.numel(), tokens,
@@ -337,7 +337,7 @@ def w4a16_moe_decode(hidden: torch.Tensor, logits: torch.Tensor, bias: torch.Ten
     x, lg = c(hidden), c(logits)
     b = c(bias) if bias is not None else None
     args = [c(t) for t in (w1_packed, w1_scales, w3_packed, w3_scales, w2_packed, w2_scales)]
-    with torch.cuda.device(dev):
+    with _w._on(dev):
         _lib.call("lk_w4a16_moe_decode", x.data_ptr(), lg.data_ptr(),
                   b.data_ptr() if b is not None else None, *(t.data_ptr() for t in args),
                   y.data_ptr(), idx.data_ptr(), w.data_ptr(), act.data_ptr(), tokens, e_total, h,
@@ -366,7 +366,7 @@ def w4a16_moe_gateup(hidden: torch.Tensor, logits: torch.Tensor, bias: torch.Ten
     x, lg = c(hidden), c(logits)
     b = c(bias) if bias is not None else None
     args = [c(t) for t in (w1_packed, w1_scales, w3_packed, w3_scales)]
-    with torch.cuda.device(dev):
+    with _w._on(dev):
         _lib.call("lk_w4a16_moe_gateup", x.data_ptr(), lg.data_ptr(),
                   b.data_ptr() if b is not None else None, *(t.data_ptr() for t in args),
                   idx.data_ptr(), w.data_ptr(), act.data_ptr(), tokens, e_total, h, inter, top_k,

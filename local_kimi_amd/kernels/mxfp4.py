@@ -68,7 +68,7 @@ def _gemm(entry: str, activations, weight_packed, weight_scale) -> torch.Tensor:
         ws = _w.workspace(_lib.query("lk_dense_gemm_workspace", m, n, k, MXFP4_GROUP_SIZE, 1, 1),
                           activations.device)
         args += [ws.data_ptr(), ws.numel()]
-    with torch.cuda.device(activations.device):
+    with _w._on(activations.device):
         _lib.call(entry, *args, _w._stream(activations.device))
     return out
 
@@ -138,7 +138,7 @@ def grouped_mxfp4_gemm(activations, expert_indices, packed, scale) -> torch.Tens
     if t == 0:
         return out
     x, idx, p, s = (_w._c(a) for a in (activations, expert_indices, packed, scale))
-    with torch.cuda.device(x.device):
+    with _w._on(x.device):
         ws = _w.workspace(_lib.query("lk_w4a16_grouped_gemm_workspace", t, r, e), x.device)
         _lib.call("lk_mxfp4_grouped_gemm", x.data_ptr(), idx.data_ptr(), p.data_ptr(),
                   s.data_ptr(), out.data_ptr(), t, r, e, n, k, ws.data_ptr(), ws.numel(),
@@ -158,7 +158,7 @@ def grouped_mxfp4_swiglu_gemm(activations, expert_indices, w1_packed, w1_scale, 
         return out
     x, idx = _w._c(activations), _w._c(expert_indices)
     banks = [_w._c(a) for a in (w1_packed, w1_scale, w3_packed, w3_scale)]
-    with torch.cuda.device(x.device):
+    with _w._on(x.device):
         ws = _w.workspace(_lib.query("lk_w4a16_grouped_gemm_workspace", t, r, e), x.device)
         _lib.call("lk_mxfp4_swiglu_gemm", x.data_ptr(), idx.data_ptr(),
                   *(b.data_ptr() for b in banks), out.data_ptr(), t, r, e, n, k, ws.data_ptr(),
@@ -182,7 +182,7 @@ def split_activations_fp8(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor, 
     lo = torch.empty((m, k), dtype=torch.uint8, device=x.device)
     sc = torch.empty((m, k // MXFP4_GROUP_SIZE), dtype=torch.int16, device=x.device)
     if m:
-        with torch.cuda.device(x.device):
+        with _w._on(x.device):
             _lib.call("lk_mxfp4_split_activations", xc.data_ptr(), hi.data_ptr(), lo.data_ptr(),
                       sc.data_ptr(), m, k, _w._stream(x.device))
     return hi, lo, sc
@@ -219,7 +219,7 @@ def mxfp4_moe_block(hidden, logits, bias, w1_packed, w1_scale, w3_packed, w3_sca
     x, lg = _w._c(hidden), _w._c(logits)
     b = _w._c(bias) if bias is not None else None
     banks = [_w._c(a) for a in (w1_packed, w1_scale, w3_packed, w3_scale, w2_packed, w2_scale)]
-    with torch.cuda.device(dev):
+    with _w._on(dev):
         ws = _w.workspace(_lib.query("lk_mxfp4_moe_forward_workspace", tokens, e1, h, inter,
                                      top_k), dev)
         _lib.call("lk_mxfp4_moe_forward", x.data_ptr(), lg.data_ptr(),
@@ -260,7 +260,7 @@ def mxfp4_expert_mlp(hidden_states: torch.Tensor, weights, *, situ_beta: float =
     lb = -1.0 if situ_linear_beta is None else float(situ_linear_beta)
     if situ_linear_beta is not None and situ_linear_beta <= 0:
         raise ValueError("situ_linear_beta must be positive or None")
-    with torch.cuda.device(dev):
+    with _w._on(dev):
         _lib.call("lk_mxfp4_expert_mlp", x.data_ptr(), *(a.data_ptr() for a in mats), y.data_ptr(),
                   act.data_ptr(), m, h, i, float(situ_beta), lb, _w._stream(dev))
     return y

@@ -68,7 +68,7 @@ def rms_norm(hidden_states: torch.Tensor, weight: torch.Tensor, eps: float) -> t
     out = torch.empty(hidden_states.shape, dtype=_result_dtype(x, w), device=x.device)
     rows = x.numel() // width
     if rows:
-        with torch.cuda.device(x.device):
+        with _w._on(x.device):
             _lib.call("lk_rms_norm", x.data_ptr(), w.data_ptr(), out.data_ptr(), rows, width,
                       float(eps), xc, wc, _w._stream(x.device))
     return out
@@ -94,7 +94,7 @@ def add_rms_norm(residual: torch.Tensor, delta: torch.Tensor, weight: torch.Tens
     out = torch.empty(residual.shape, dtype=_result_dtype(r, w), device=r.device)
     rows = r.numel() // width
     if rows:
-        with torch.cuda.device(r.device):
+        with _w._on(r.device):
             _lib.call("lk_add_rms_norm", r.data_ptr(), d.data_ptr(), w.data_ptr(),
                       hidden.data_ptr(), out.data_ptr(), rows, width, float(eps), xc, wc,
                       _w._stream(r.device))
@@ -128,7 +128,7 @@ def rms_gated_norm(values: torch.Tensor, gate: torch.Tensor, weight: torch.Tenso
     out = torch.empty(values.shape, dtype=in_dtype, device=v.device)
     rows = v.numel() // width
     if rows:
-        with torch.cuda.device(v.device):
+        with _w._on(v.device):
             _lib.call("lk_rms_gated_norm", v.data_ptr(), g.data_ptr(), w.data_ptr(),
                       out.data_ptr(), rows, width, float(eps), vc, ic, gc, wc,
                       _w._stream(v.device))

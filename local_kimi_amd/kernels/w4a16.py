@@ -13,13 +13,32 @@ engine/quant/w4a16.py:14). Here it is read from the scale tensor's last axis:
 
 from __future__ import annotations
 
+import contextlib
+
 import torch
 
 from .. import _lib
 
 
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(device: torch.device) -> int:
+    """The current stream's handle on ``device`` (a CUDA tensor's device)."""
+    if _raw_stream is not None and device.index is not None:
+        return _raw_stream(device.index)  # no Stream object per call
     return torch.cuda.current_stream(device).cuda_stream
+
+
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def _on(device: torch.device):
+    """``torch.cuda.device(device)``, or nothing where it is already current
+    (the context costs a few microseconds, most of a decode launch)."""
+    if device.index == torch.cuda.current_device():
+        return _SAME_DEVICE
+    return torch.cuda.device(device)
 
 
 def _group_size(reduction: int, scale_columns: int, what: str) -> int:
@@ -99,7 +118,7 @@ def _dense(entry: str, activations, packed_weights, scales):
     if m == 0:
         return out
     x, p, s = _c(activations), _c(packed_weights), _c(scales)
-    with torch.cuda.device(activations.device):
+    with _on(activations.device):
         _lib.call(entry, x.data_ptr(), p.data_ptr(), s.data_ptr(), out.data_ptr(), m, n, k, g,
                   _stream(activations.device))
     return out
@@ -114,7 +133,7 @@ def _dense_gemm(activations, packed_weights, scales):
         return out
     ws = workspace(_lib.query("lk_dense_gemm_workspace", m, n, k, g, 1, 0), activations.device)
     x, p, s = _c(activations), _c(packed_weights), _c(scales)
-    with torch.cuda.device(activations.device):
+    with _on(activations.device):
         _lib.call("lk_w4a16_dense_gemm_ws", x.data_ptr(), p.data_ptr(), s.data_ptr(),
                   out.data_ptr(), m, n, k, g, ws.data_ptr(), ws.numel(),
                   _stream(activations.device))
@@ -185,7 +204,7 @@ def _grouped(entry: str, activations, expert_indices, packed_weights, scales):
     if t == 0:
         return out
     x, idx, p, s = _c(activations), _c(expert_indices), _c(packed_weights), _c(scales)
-    with torch.cuda.device(activations.device):
+    with _on(activations.device):
         if entry.endswith("_gemm"):
             ws = workspace(_lib.query("lk_w4a16_grouped_gemm_workspace", t, r, e), x.device)
             _lib.call(entry, x.data_ptr(), idx.data_ptr(), p.data_ptr(), s.data_ptr(),
@@ -252,7 +271,7 @@ def _swiglu(gemm: bool, activations, expert_indices, w1_packed, w1_scales, w3_pa
     p1, s1, p3, s3 = _c(w1_packed), _c(w1_scales), _c(w3_packed), _c(w3_scales)
     args = [x.data_ptr(), idx.data_ptr(), p1.data_ptr(), s1.data_ptr(), p3.data_ptr(),
             s3.data_ptr(), out.data_ptr(), t, r, e, n, k, g]
-    with torch.cuda.device(activations.device):
+    with _on(activations.device):
         if gemm:
             ws = workspace(_lib.query("lk_w4a16_grouped_gemm_workspace", t, r, e), x.device)
             _lib.call("lk_w4a16_swiglu_gemm", *args, ws.data_ptr(), ws.numel(),
@@ -288,7 +307,7 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
         raise ValueError("silu_mul requires CUDA tensors on one device")
     out = torch.empty_like(gate, memory_format=torch.contiguous_format)
     g, u = _c(gate), _c(up)
-    with torch.cuda.device(gate.device):
+    with _on(gate.device):
         _lib.call("lk_silu_mul", g.data_ptr(), u.data_ptr(), out.data_ptr(), gate.numel(),
                   _stream(gate.device))
     return out
@@ -345,7 +364,7 @@ def fused_w2_combine(activated, expert_indices, combine_weights, w2_packed, w2_s
         return out
     a, idx, cw = _c(activated), _c(expert_indices), _c(combine_weights)
     p, s = _c(w2_packed), _c(w2_scales)
-    with torch.cuda.device(activated.device):
+    with _on(activated.device):
         _lib.call("lk_w4a16_w2_combine", a.data_ptr(), idx.data_ptr(), cw.data_ptr(), p.data_ptr(),
                   s.data_ptr(), out.data_ptr(), t, r, e, h, i, g, _stream(activated.device))
     return out
@@ -362,7 +381,7 @@ def route_combine(expert_outputs: torch.Tensor, combine_weights: torch.Tensor) -
     t, r, h = expert_outputs.shape
     out = torch.empty((t, h), dtype=torch.bfloat16, device=expert_outputs.device)
     eo, cw = _c(expert_outputs), _c(combine_weights)
-    with torch.cuda.device(expert_outputs.device):
+    with _on(expert_outputs.device):
         _lib.call("lk_route_combine", eo.data_ptr(), cw.data_ptr(), out.data_ptr(), t, r, h,
                   _stream(expert_outputs.device))
     return out
@@ -425,8 +444,13 @@ def fused_qkv_w4a16(activations, q_packed, q_scales, k_packed, k_scales, v_packe
         return tuple(outs)
     x = _c(activations)
     w = [_c(t) for t in (q_packed, q_scales, k_packed, k_scales, v_packed, v_scales)]
+    if m < DENSE_GEMM_MIN_ROWS:  # the GEMV launch takes no workspace
+        with _on(dev):
+            _lib.call("lk_w4a16_fused_qkv", x.data_ptr(), *(t.data_ptr() for t in w),
+                      *(o.data_ptr() for o in outs), m, n, k, g, _stream(dev))
+        return tuple(outs)
     ws = workspace(_lib.query("lk_dense_gemm_workspace", m, n, k, g, 3, 0), dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _lib.call("lk_w4a16_fused_qkv_ws", x.data_ptr(), *(t.data_ptr() for t in w),
                   *(o.data_ptr() for o in outs), m, n, k, g, ws.data_ptr(), ws.numel(),
                   _stream(dev))
