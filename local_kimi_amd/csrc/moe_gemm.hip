@@ -3435,6 +3435,10 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
     d.a_lo = as.lo;
     d.a_sc = as.sc;
     d.a_rows = entries;
+    // the gate/up launch has routed: the down GEMM reads the tables it wrote,
+    // so the routing scratch is no part of what this launch needs of the LDS
+    d.rt_logits = nullptr;
+    d.rt_from_idx = 0;
     if (paired) {  // written paired by the gate/up GEMM, with their group sums
       d.a_pair = act;
       d.a_neg = d.out_neg;

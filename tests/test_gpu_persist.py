@@ -293,3 +293,26 @@ def test_moe_block_narrow_groups_match_per_tile_and_oracle(rng, monkeypatch, gro
 
     moved = (args[0], args[1], None, *(shifted(b) for b in dev_banks), k, 2.446)
     assert torch.equal(w4a16_moe_forward(*moved)[0], y)
+
+
+@pytest.mark.parametrize("group", [32, 128])
+@pytest.mark.parametrize("tokens,inter", [(40, 512), (100, 1024), (113, 512)])
+def test_ranking_gate_up_with_a_narrow_down_gemm(rng, monkeypatch, group, tokens, inter):
+    """256 routed experts: the gate/up GEMM's routing scratch (up to 77 KB at 113
+    tokens) fits the LDS of k = 2304 and not that of the down GEMM's k, which
+    needs none of it."""
+    from local_kimi_amd.kernels import w4a16_moe_forward
+    from local_kimi_amd.workloads import zipf_router_logits
+
+    e_routed, h, k = 256, 2304, 8
+    gen = torch.Generator(device=DEV).manual_seed(20260803 + tokens)
+    banks = (*_gpu_w4_bank(gen, e_routed + 1, inter, h, group),
+             *_gpu_w4_bank(gen, e_routed + 1, inter, h, group),
+             *_gpu_w4_bank(gen, e_routed + 1, h, inter, group))
+    x = random_bf16_bits(rng, (tokens, h))
+    logits = zipf_router_logits(rng, tokens, e_routed)
+    args = (_dev(x), _dev(logits), None, *banks, k, 2.446)
+    (y, idx, w), (y0, idx0, w0) = _both(monkeypatch, w4a16_moe_forward, *args)
+    assert torch.equal(idx, idx0) and torch.equal(w, w0)
+    assert torch.equal(y, y0), "persistent and per-tile kernels differ"
+    assert np.array_equal(idx.cpu().numpy(), OM.route(logits, None, k, routed_scaling_factor=2.446)[0])
