@@ -31,6 +31,7 @@
 
 #include <initializer_list>
 #include <mutex>
+#include <type_traits>
 
 #include "lk_gemm.hpp"
 #include "lk_route.hpp"
@@ -2600,15 +2601,24 @@ int persist_depth(const GemmArgs& g, int nbuf, size_t lds, int64_t tiles_bound, 
                   bool launch) {
   // the ring depth divides the k-steps (at least one whole round per unit)
   const int64_t ksteps = g.k / 128;
-  if (ksteps >= 6 && ksteps % 6 == 0)
-    return persist_one<FMT, MATS, 6, GATHER, SCATTER, SPLIT, SWI, ROUTED>(g, nbuf, lds,
-                                                                          tiles_bound, s, launch);
-  if (ksteps >= 8 && ksteps % 8 == 0)
-    return persist_one<FMT, MATS, 8, GATHER, SCATTER, SPLIT, SWI, ROUTED>(g, nbuf, lds,
-                                                                          tiles_bound, s, launch);
-  if (ksteps >= 4 && ksteps % 4 == 0)
-    return persist_one<FMT, MATS, 4, GATHER, SCATTER, SPLIT, SWI, ROUTED>(g, nbuf, lds,
-                                                                          tiles_bound, s, launch);
+  // Two matrices at groups of 32 or 64: four k-steps of ring wherever they
+  // divide, since a deeper one does not fit the registers (spilled registers at
+  // 4, 6 and 8 k-steps: 13, 145, 239 at G = 32, none, 1, 59 at G = 64). Gate/up
+  // of 64 tokens x 8 routes over 256 experts, 1024 x 2048, in us: G = 32 537 at
+  // eight, 131 at four (per-tile kernel 463), G = 64 146 at eight, 112 at four;
+  // k = 3072 over 64 experts 165 at six, 52 at four. Six stays where four does
+  // not divide (k = 2304, 256 experts: G = 32 406, per-tile 440).
+  constexpr bool kShallow = MATS == 2 && (FMT == kFmtW4G32 || FMT == kFmtW4G64);
+  auto one = [&](auto depth) {
+    return persist_one<FMT, MATS, decltype(depth)::value, GATHER, SCATTER, SPLIT, SWI, ROUTED>(
+        g, nbuf, lds, tiles_bound, s, launch);
+  };
+  if (kShallow && ksteps >= 4 && ksteps % 4 == 0) return one(std::integral_constant<int, 4>{});
+  if (ksteps >= 6 && ksteps % 6 == 0) return one(std::integral_constant<int, 6>{});
+  if constexpr (!kShallow) {
+    if (ksteps >= 8 && ksteps % 8 == 0) return one(std::integral_constant<int, 8>{});
+  }
+  if (ksteps >= 4 && ksteps % 4 == 0) return one(std::integral_constant<int, 4>{});
   return -1;
 }
 
