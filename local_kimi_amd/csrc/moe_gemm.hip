@@ -3477,10 +3477,14 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
       path_choice(kKnobMoeSplitSwiglu) != 1 &&
       persist_fmt<1>(mx, g, Mode::Gather, tb, s, "", PsForm::SplitGateUp, false) == 0 &&
       persist_fmt<1>(mx, down_args(g), Mode::Scatter, tb, s, "", PsForm::SwiDown, false) == 0;
-  // G = 32 at widths of the persistent kernels: their two-matrix gate/up unit,
-  // which the token-major W2 follows, does not fit the registers (4 tokens of
-  // the Kimi-Linear layer 73 us with it, 41 with the split form)
-  if (group == 32 && h % 256 == 0 && i % 256 == 0) w2_rows = false;
+  // G = 32: where the split form applies and the gate/up unit of two matrices,
+  // which the token-major W2 follows, is left a ring of six k-steps that
+  // spills (h / 128 not a multiple of 4), the split form is the faster one: 4
+  // tokens of the Kimi-Linear layer (h = 2304) 42 us against 73. With four
+  // k-steps of ring the token-major tail stays ahead (256 experts, 2048 x 1024,
+  // 4 tokens 37 against 40 us), and where no split form applies it is all there
+  // is to gain: 2304 x 1280, 3 tokens 67 us with it, 99 without.
+  if (group == 32 && split_fits && h % 512 != 0) w2_rows = false;
   const bool split = split_fits && !w2_rows;
   const Mode gu_mode = w2_rows ? Mode::GatherScatter : Mode::Gather;
   // Batches of at most 8 tokens (one per wave) on the persistent 16-row

@@ -316,3 +316,35 @@ def test_ranking_gate_up_with_a_narrow_down_gemm(rng, monkeypatch, group, tokens
     assert torch.equal(idx, idx0) and torch.equal(w, w0)
     assert torch.equal(y, y0), "persistent and per-tile kernels differ"
     assert np.array_equal(idx.cpu().numpy(), OM.route(logits, None, k, routed_scaling_factor=2.446)[0])
+
+
+@pytest.mark.parametrize("group", [32, 64])
+@pytest.mark.parametrize("h,inter,tokens", [(1280, 512, 3), (768, 1280, 2), (512, 512, 4),
+                                            (768, 512, 1)])
+def test_few_tokens_end_in_the_token_major_w2_launch(rng, group, h, inter, tokens):
+    """Up to 4 tokens end in the token-major W2 + combine, which sums over the
+    intermediate in another order than the down GEMM: the block is that launch's
+    bits on the same activations, except at G = 32 where the split SwiGLU takes
+    the call (h / 128 not a multiple of 4, both its launches applying), and it
+    matches the oracle everywhere."""
+    from local_kimi_amd.kernels import fused_w2_combine, grouped_w4a16_swiglu_gemm, w4a16_moe_forward
+
+    e_routed, k = 24, 4
+    banks = (*_w4_bank(rng, e_routed + 1, inter, h, group),
+             *_w4_bank(rng, e_routed + 1, inter, h, group),
+             *_w4_bank(rng, e_routed + 1, h, inter, group))
+    x = random_bf16_bits(rng, (tokens, h))
+    logits = rng.normal(0, 1, (tokens, e_routed)).astype(np.float32)
+    dev = [_dev(b) for b in banks]
+    y, idx, w = w4a16_moe_forward(_dev(x), _dev(logits), None, *dev, k, 2.446)
+    ey, eidx, _ = OM.moe_block(x, logits, None, *banks, top_k=k, routed_scaling_factor=2.446,
+                               group_size=group)
+    assert np.array_equal(idx.cpu().numpy(), eidx)
+    assert_close_bf16(to_bits(y), ey, what=f"G={group} h={h} i={inter} T={tokens}")
+    if group == 32 and (h, inter) == (768, 512):  # the split form
+        return
+    stable = torch.cat((idx, torch.full((tokens, 1), e_routed, device=DEV)), 1)
+    act = grouped_w4a16_swiglu_gemm(_dev(x), stable, *dev[:4])
+    cw = torch.cat((w, torch.ones((tokens, 1), device=DEV)), 1)
+    want = fused_w2_combine(act, stable, cw, *dev[4:])
+    assert torch.equal(y, want), "not the token-major W2 launch"
