@@ -317,9 +317,12 @@ LK_API int lk_w4a16_moe_forward(const uint16_t* x, const float* logits, const fl
  * loops and harnesses that forbid hipMalloc: the same arguments minus the
  * workspace, which here is a static device array of
  * lk_w4a16_moe_forward_static_capacity() bytes (12 MiB) per GPU, held until
- * the process ends. Calls whose lk_w4a16_moe_forward_workspace() exceeds it
- * are rejected before anything is launched (up to 160 tokens at the
- * Kimi-Linear shape: hidden 2304, intermediate 1024, 257 experts, top-8).
+ * the process ends. Calls that need more are rejected before anything is
+ * launched (up to 160 tokens at the Kimi-Linear shape: hidden 2304,
+ * intermediate 1024, 257 experts, top-8). Above 2048 token-routes
+ * lk_w4a16_moe_forward_workspace() is up to 3 % more than a call needs; a
+ * call at groups of 32 or 64 that gets no more than its need stages its rows
+ * unpaired (the same bits).
  * Nothing is allocated or freed; the scratch needs no clearing (every table
  * and row in it is written before it is read). Every call on one GPU shares
  * that GPU's array: calls that overlap on one GPU (two streams, two host

@@ -2306,7 +2306,8 @@ SplitBufs split_bufs(char* base, int64_t elems) {
 }
 
 MoeLayout moe_layout(int64_t entries, int64_t experts, int64_t act_cols, int64_t out_cols,
-                     int64_t split_x_elems = 0, int64_t pair_rows = 0, int act_mult = 1) {
+                     int64_t split_x_elems = 0, int64_t pair_rows = 0, int act_mult = 1,
+                     int pair_sums = 1) {
   MoeLayout l;
   l.sched = sched_layout(entries, experts);
   size_t at = l.sched.total;
@@ -2335,14 +2336,15 @@ MoeLayout moe_layout(int64_t entries, int64_t experts, int64_t act_cols, int64_t
   if (split_x_elems > 0) at += split_bytes(entries * act_cols);
   // W4A16 64-row launches: the gathered input (pair_rows rows of out_cols)
   // paired for direct loads, its group sums and the activations' group sums
-  // (the gate/up GEMM writes the activations paired in place)
+  // (the gate/up GEMM writes the activations paired in place): pair_sums
+  // floats per 128-wide k-step
   const bool pairs = pair_rows > 0;
   l.x_pair = at;
   if (pairs) at += align_up(static_cast<size_t>(pair_rows) * out_cols * 2);
   l.x_neg = at;
-  if (pairs) at += align_up(static_cast<size_t>(pair_rows) * (out_cols / 128) * 16);
+  if (pairs) at += align_up(static_cast<size_t>(pair_rows) * (out_cols / 128) * 4 * pair_sums);
   l.act_neg = at;
-  if (pairs) at += align_up(static_cast<size_t>(entries) * (act_cols / 128) * 16);
+  if (pairs) at += align_up(static_cast<size_t>(entries) * (act_cols / 128) * 4 * pair_sums);
   l.total = at;
   return l;
 }
@@ -2855,14 +2857,28 @@ int stream_tile_mt(int64_t entries) {
 
 // Whether an expert-major W4A16 call of `entries` token-routes sizes the
 // paired-activation buffers of its 64-row launches into the workspace (the
-// workspace query and the call agree through this; calls whose group is not
-// 128 leave them unused).
+// workspace query and the call agree through this).
 bool moe_pairs(int64_t entries, bool mx) { return !mx && stream_tile_mt(entries) == 4; }
 
 // Whether an expert-major call of `entries` token-routes sizes its activation
 // region for the split SwiGLU of the 16-row launches ([gate | up] rows, twice
 // the SwiGLU's width); the workspace query and the call agree through this.
 int moe_act_mult(int64_t entries) { return stream_tile_mt(entries) == 1 ? 2 : 1; }
+
+// Group sums of a paired k-step: one float at G = 128, four at G = 32 and 64.
+// The workspace query, which knows no group, asks for four; a call takes a
+// workspace (and the static scratch) sized for one, the size before groups of
+// 32 and 64 were paired, and then stages those groups' rows unpaired.
+constexpr int kPairSumsMax = 4;
+int pair_sums_per_step(int64_t group) { return group == 128 ? 1 : kPairSumsMax; }
+
+// Layout of a W4A16 block of `tokens` tokens.
+MoeLayout w4_moe_layout(int64_t tokens, int64_t experts, int64_t h, int64_t i, int64_t top_k,
+                        int pair_sums) {
+  const int64_t entries = tokens * (top_k + 1);
+  return moe_layout(entries, experts, i, h, 0, moe_pairs(entries, false) ? tokens : 0,
+                    moe_act_mult(entries), pair_sums);
+}
 
 template <int MATS>
 int persist_fmt(bool mx, const GemmArgs& g, Mode mode, int64_t tiles_bound, hipStream_t s,
@@ -2894,7 +2910,7 @@ void dense_args(GemmArgs& g, const uint16_t* x, int64_t m, int64_t n, int64_t k,
 
 // Group sums of one paired row (pair_rows_kernel): a float per 128-wide k-step
 // at G = 128, four at G = 32 and 64.
-int64_t pair_sums(int64_t k, int64_t group) { return (k / 128) * (group == 128 ? 1 : 4); }
+int64_t pair_sums(int64_t k, int64_t group) { return (k / 128) * pair_sums_per_step(group); }
 
 // Workspace of a dense W4A16 product on the prefill GEMM, which loads its
 // rows directly: the rows paired in the weight decode's k order and their
@@ -3294,11 +3310,7 @@ int64_t lk_w4a16_moe_forward_workspace(int64_t tokens, int64_t experts, int64_t 
                                        int64_t top_k) {
   if (tokens < 0 || experts < 2 || h <= 0 || i <= 0 || top_k <= 0) return -1;
   if (check_schedule_dims(tokens, top_k + 1, experts)) return -1;
-  const int64_t entries = tokens * (top_k + 1);
-  return static_cast<int64_t>(moe_layout(entries, experts, i, h, 0,
-                                         moe_pairs(entries, false) ? tokens : 0,
-                                         moe_act_mult(entries))
-                                  .total);
+  return static_cast<int64_t>(w4_moe_layout(tokens, experts, h, i, top_k, kPairSumsMax).total);
 }
 
 int64_t lk_mxfp4_moe_forward_workspace(int64_t tokens, int64_t experts, int64_t h, int64_t i,
@@ -3348,11 +3360,13 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
   LK_REQUIRE(x && logits && workspace, "null pointer argument");
   const int64_t routes = top_k + 1;
   const int64_t entries = tokens * routes;
-  const MoeLayout l = moe_layout(entries, experts, i, h, mx ? tokens * h : 0,
-                                 moe_pairs(entries, mx) ? tokens : 0, moe_act_mult(entries));
-  LK_REQUIRE(workspace_bytes >= static_cast<int64_t>(l.total),
-             "MoE workspace too small: %lld < %lld bytes", (long long)workspace_bytes,
-             (long long)l.total);
+  const MoeLayout l = mx ? moe_layout(entries, experts, i, h, tokens * h, 0, moe_act_mult(entries))
+                         : w4_moe_layout(tokens, experts, h, i, top_k,
+                                         pair_sums_per_step(group_size));
+  const int64_t least = static_cast<int64_t>(
+      mx ? l.total : w4_moe_layout(tokens, experts, h, i, top_k, 1).total);
+  LK_REQUIRE(workspace_bytes >= least, "MoE workspace too small: %lld < %lld bytes",
+             (long long)workspace_bytes, (long long)least);
   hipStream_t s = as_stream(stream);
   char* ws = static_cast<char*>(workspace);
   auto* offsets = reinterpret_cast<int32_t*>(ws + l.offsets);
@@ -3375,7 +3389,8 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
   const int fmt = mx ? kFmtMxBf16 : kFmtW4A16;
   const bool tile = mt == 4 && !f8 && tile_format(fmt, group) >= 0 && h % 128 == 0 && i % 128 == 0 &&
                     i * h <= kMaxDirectBytes &&
-                    tile_aligned({x, w1_packed, w3_packed, w2_packed},
+                    workspace_bytes >= static_cast<int64_t>(l.total) &&
+                    tile_aligned({x, w1_packed, w3_packed, w2_packed, workspace},
                                  {w1_scales, w3_scales, w2_scales});
   // W4A16 on 64-row tiles: x and the activations go in paired
   const bool paired = !mx && tile;
@@ -3674,7 +3689,9 @@ int lk_w4a16_moe_forward_static(const uint16_t* x, const float* logits, const fl
                                 int64_t experts, int64_t h, int64_t i, int64_t top_k,
                                 float routed_scaling_factor, int renormalize, int64_t group_size,
                                 void* stream) {
-  const int64_t need = lk_w4a16_moe_forward_workspace(tokens, experts, h, i, top_k);
+  const bool valid = lk_w4a16_moe_forward_workspace(tokens, experts, h, i, top_k) >= 0;
+  const int64_t need =
+      valid ? static_cast<int64_t>(w4_moe_layout(tokens, experts, h, i, top_k, 1).total) : -1;
   LK_REQUIRE(need >= 0, "invalid MoE dimensions (tokens %lld, experts %lld, top_k %lld)",
              (long long)tokens, (long long)experts, (long long)top_k);
   LK_REQUIRE(need <= static_cast<int64_t>(kStaticScratchBytes),

@@ -91,3 +91,66 @@ def test_static_scratch_refuses_calls_past_its_size(banks):
     x, logits = _inputs(np.random.default_rng(1), too_many)
     with pytest.raises(RuntimeError, match="static scratch holds"):
         _run(True, x, logits, banks)
+
+
+def _small_call(group, routed, top_k, tokens, h, inter, seed):
+    """A block of random weights: run(static, shift) -> (y, idx, w), the
+    workspace `shift` bytes off the allocator's alignment."""
+    from local_kimi_amd.quant import quantise
+
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+
+    def bank(n, k):
+        enc = [quantise((torch.randn(n, k, device=DEV, generator=gen) * 0.02).to(torch.bfloat16),
+                        group_size=group) for _ in range(routed + 1)]
+        return torch.stack([e.packed for e in enc]), torch.stack([e.scales for e in enc])
+
+    weights = (*bank(inter, h), *bank(inter, h), *bank(h, inter))
+    x = torch.randn(tokens, h, device=DEV, generator=gen).to(torch.bfloat16)
+    logits = torch.randn(tokens, routed, device=DEV, generator=gen)
+    need = _lib.query("lk_w4a16_moe_forward_workspace", tokens, routed + 1, h, inter, top_k)
+
+    def run(static, shift=0):
+        y = torch.full((tokens, h), float("nan"), dtype=torch.bfloat16, device=DEV)
+        idx = torch.empty((tokens, top_k), dtype=torch.long, device=DEV)
+        w = torch.empty((tokens, top_k), dtype=torch.float32, device=DEV)
+        ws = torch.empty((need + 16,), dtype=torch.uint8, device=DEV)
+        args = [x.data_ptr(), logits.data_ptr(), None, *(b.data_ptr() for b in weights),
+                y.data_ptr(), idx.data_ptr(), w.data_ptr()]
+        entry = "lk_w4a16_moe_forward_static" if static else "lk_w4a16_moe_forward"
+        _lib.call(entry, *args, *(() if static else (ws.data_ptr() + shift, need)), tokens,
+                  routed + 1, h, inter, top_k, 2.446, 1, group,
+                  torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        return y, idx, w
+
+    return run
+
+
+@pytest.mark.parametrize("group", [32, 128])
+def test_static_scratch_at_the_edge_of_its_size(banks, group):
+    """Past 2048 token-routes the rows are paired, and groups of 32 take three
+    floats more per row and k-step for it than groups of 128. The scratch takes
+    every call that it held without them (staged unpaired, the same bits)."""
+    h = inter = 512
+    routed, top_k = 24, 4
+    cap = _lib.query("lk_w4a16_moe_forward_static_capacity")
+
+    def query(t):
+        return _lib.query("lk_w4a16_moe_forward_workspace", t, routed + 1, h, inter, top_k)
+
+    def sums(t):  # what the query holds beyond one float per row and k-step
+        return 12 * (h // 128) * t + 12 * (inter // 128) * t * (top_k + 1)
+
+    tokens = max(t for t in range(410, 1600) if query(t) - sums(t) + 1024 <= cap)
+    assert query(tokens) > cap
+    run = _small_call(group, routed, top_k, tokens, h, inter, 7)
+    for a, b in zip(run(True), run(False)):
+        assert torch.equal(a, b)
+
+
+def test_workspace_off_its_alignment(banks):
+    """A workspace at 4 bytes off, which the direct loads do not take."""
+    run = _small_call(32, 8, 4, 420, 256, 256, 9)
+    for a, b in zip(run(False), run(False, 4)):
+        assert torch.equal(a, b)
