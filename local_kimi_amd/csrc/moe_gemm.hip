@@ -2407,13 +2407,15 @@ int schedule_launch(const RouteTable& rt, int64_t entries, char* ws, const Sched
   return check_launch("moe schedule");
 }
 
+constexpr int64_t kMaxPairUnits = int64_t{1} << 27;  // rows x k-steps of one pairing launch
+
 // Paired copy + group sums of `rows` bf16 rows of k (k % 128 == 0) for the
 // direct-load W4A16 GEMM.
 int pair_rows_launch(const uint16_t* x, uint16_t* xp, float* neg, int64_t rows, int64_t k,
                      int64_t group, hipStream_t s) {
   const int64_t units = rows * (k / 128);
   if (units == 0) return LK_OK;
-  LK_REQUIRE(k % 128 == 0 && units < (1LL << 27), "pairing: unsupported size");
+  LK_REQUIRE(k % 128 == 0 && units < kMaxPairUnits, "pairing: unsupported size");
   const unsigned nb = static_cast<unsigned>((units * 16 + 255) / 256);
   const uint32_t n = static_cast<uint32_t>(units);
   if (group == 32) pair_rows_kernel<1><<<nb, 256, 0, s>>>(x, xp, neg, n);
@@ -2428,7 +2430,7 @@ int route_pair_launch(const float* logits, const float* bias, int64_t* idx, floa
                       int64_t tokens, int64_t routed, int64_t top_k, float scaling, int renorm,
                       const uint16_t* x, uint16_t* xp, float* neg, int64_t k, int64_t group,
                       hipStream_t s) {
-  LK_REQUIRE(k % 128 == 0 && tokens * (k / 128) < (1LL << 27) && routed <= 256 &&
+  LK_REQUIRE(k % 128 == 0 && tokens * (k / 128) < kMaxPairUnits && routed <= 256 &&
                  tokens <= 2147483647LL,
              "router + pairing: unsupported size");
   auto* fn = group == 32   ? &route_pair_kernel<4, 1>
@@ -2778,14 +2780,20 @@ bool tile_aligned(std::initializer_list<const void*> rows_and_codes,
   return (any & 15) == 0 && (sc & 3) == 0;
 }
 
+// Whether a dense product's rows and codes lie within the prefill GEMM's 32-bit
+// byte offsets.
+bool tile_sizes(int64_t m, int64_t n, int64_t k) {
+  return m * k * 2 <= kMaxDirectBytes && n * k <= kMaxDirectBytes;
+}
+
 // Whether the prefill GEMM (tile_gemm.hip) takes a dense launch: whole 128-wide
 // k-steps, 32-bit byte offsets, paired rows (W4A16) and operands aligned for
 // its loads (what the kernels it stands in for read in 2- and 4-byte pieces
-// may lie anywhere).
+// may lie anywhere). The path knob dense_gemm=lds takes none.
 bool tile_fits(const GemmArgs& g, int fmt) {
   const int tf = tile_format(fmt, g.group);
-  if (tf < 0 || g.k % 128 != 0 || g.a_rows <= 0) return false;
-  if (g.a_rows * g.k * 2 > kMaxDirectBytes || g.n * g.k > kMaxDirectBytes) return false;
+  if (path_choice(kKnobDenseGemm) == 1 || tf < 0 || g.k % 128 != 0 || g.a_rows <= 0) return false;
+  if (!tile_sizes(g.a_rows, g.n, g.k)) return false;
   if (fmt_is_w4(tf) && !(g.a_pair && g.a_neg)) return false;
   return tile_aligned({fmt_is_w4(tf) ? g.a_pair : g.a, g.wp[0], g.wp[1], g.wp[2], g.out[0],
                        g.out[1], g.out[2]},
@@ -2801,7 +2809,7 @@ bool tile_fits(const GemmArgs& g, int fmt) {
 template <int FMT>
 int dense_launch(const GemmArgs& g, int64_t tiles, hipStream_t s, const char* what) {
   const bool lds = path_choice(kKnobDenseGemm) == 1;
-  if (!lds && tile_fits(g, FMT))
+  if (tile_fits(g, FMT))
     return tile_gemm_launch(tile_format(FMT, g.group), 1, g, Mode::Dense, tiles, s, what);
   if (!lds && stream_fits(g.k, 4, g.group, FMT != kFmtW4A16))
     return stream_launch<FMT, 1>(g, Mode::Dense, tiles, 4, s, what);
@@ -2914,9 +2922,12 @@ int64_t pair_sums(int64_t k, int64_t group) { return (k / 128) * pair_sums_per_s
 
 // Workspace of a dense W4A16 product on the prefill GEMM, which loads its
 // rows directly: the rows paired in the weight decode's k order and their
-// group sums (G <= 128, k % 128 == 0, from 16 rows); 0 where it does not apply.
+// group sums (G <= 128, k % 128 == 0, from 16 rows); 0 where it does not apply
+// (at G = 128 rows beyond the GEMM's offsets are sized too: that is what its
+// query has always answered).
 int64_t dense_pair_bytes(int64_t m, int64_t k, int64_t group) {
   if (m < 16 || (group != 32 && group != 64 && group != 128) || k % 128 != 0) return 0;
+  if (group != 128 && m * k * 2 > kMaxDirectBytes) return 0;
   return static_cast<int64_t>(align_up(static_cast<size_t>(m * k * 2)) +
                               align_up(static_cast<size_t>(m * pair_sums(k, group) * 4)));
 }
@@ -2926,6 +2937,7 @@ int64_t dense_pair_bytes(int64_t m, int64_t k, int64_t group) {
 int64_t dense_ws_bytes(bool mx, int64_t m, int64_t n, int64_t k, int64_t group, int64_t outputs) {
   const int64_t pairs = mx ? 0 : dense_pair_bytes(m, k, group);
   if (k % 128 != 0 || m < 1 || (!mx && pairs == 0)) return pairs;
+  if (!tile_sizes(m, n, k)) return group == 128 ? pairs : 0;
   return pairs + tile_gemm_split_bytes(mx, m, n, k, outputs);
 }
 
@@ -2939,9 +2951,11 @@ void dense_split(GemmArgs& g, bool mx, int64_t group, void* workspace, int64_t w
     g.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + pairs);
 }
 
-// The pre-pass of the direct form: pairs x into the workspace and points the
+// The pre-pass of the direct form, for a launch whose other operands are set:
+// where the prefill GEMM takes it, pairs x into the workspace and points the
 // launch at it. At G = 32 and 64 a call without the workspace keeps the
-// staged form, which needs none.
+// staged form, which needs none; so does every launch that the GEMM does not
+// take, without the pass over its rows.
 int dense_pairs(GemmArgs& g, const uint16_t* x, int64_t m, int64_t k, int64_t group,
                 void* workspace, int64_t workspace_bytes, hipStream_t s, const char* what) {
   const int64_t need = dense_pair_bytes(m, k, group);
@@ -2950,14 +2964,16 @@ int dense_pairs(GemmArgs& g, const uint16_t* x, int64_t m, int64_t k, int64_t gr
   if (!have && group != 128) return LK_OK;
   LK_REQUIRE(have, "%s: workspace too small: %lld < %lld bytes", what, (long long)workspace_bytes,
              (long long)need);
-  auto* xp = static_cast<uint16_t*>(workspace);
-  auto* neg = reinterpret_cast<float*>(static_cast<char*>(workspace) +
-                                       align_up(static_cast<size_t>(m * k * 2)));
-  if (int rc = pair_rows_launch(x, xp, neg, m, k, group, s)) return rc;
-  g.a_pair = xp;
-  g.a_neg = neg;
-  g.a_rows = m;
-  return LK_OK;
+  LK_REQUIRE(m * (k / 128) < kMaxPairUnits, "%s: too many rows to pair", what);
+  GemmArgs paired = g;
+  paired.a_pair = static_cast<uint16_t*>(workspace);
+  paired.a_neg = reinterpret_cast<float*>(static_cast<char*>(workspace) +
+                                          align_up(static_cast<size_t>(m * k * 2)));
+  paired.a_rows = m;
+  if (!tile_fits(paired, kFmtW4A16)) return LK_OK;
+  g = paired;
+  return pair_rows_launch(x, const_cast<uint16_t*>(g.a_pair), const_cast<float*>(g.a_neg), m, k,
+                          group, s);
 }
 
 }  // namespace

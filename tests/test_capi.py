@@ -90,6 +90,19 @@ def test_dense_workspace_sizes_and_refusals(lib):
                   None, 0, None)
 
 
+def test_dense_workspace_covers_only_what_the_prefill_gemm_takes(lib):
+    """Rows or codes beyond 32-bit byte offsets stay on the staged kernels, so at
+    groups of 32 and 64 (and for MXFP4) nothing is asked for them; groups of 128
+    keep the answer of their own query."""
+    sizes = [(1 << 22, 256, 1024), (1 << 20, 32, 16384), (64, 1 << 20, 8192)]
+    for m, n, k in sizes:
+        for group, mx in ((32, 0), (64, 0), (32, 1)):
+            assert lib.lk_dense_gemm_workspace(m, n, k, group, 1, mx) == 0
+        assert lib.lk_dense_gemm_workspace(m, n, k, 128, 1, 0) == \
+            lib.lk_w4a16_dense_gemm_workspace(m, k, 128)
+    assert lib.lk_dense_gemm_workspace(1 << 20, 256, 1024, 32, 1, 0) > (1 << 31)
+
+
 def test_grouped_router_argument_errors(lib):
     # (logits, bias, idx, w, tokens, experts, top_k, groups, topk_group, scale, renorm, stream)
     with pytest.raises(RuntimeError, match="divisible"):

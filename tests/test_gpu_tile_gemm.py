@@ -179,3 +179,46 @@ def test_fused_qkv_and_mxfp4_split_over_k_match_oracle(rng):
     y = mxfp4_gemm(torch.from_numpy(xh).to(DEV), _dev(p), _dev(s)).float().cpu().numpy()
     want = xh.astype(np.float64) @ X.dequantize(p, s).astype(np.float64).T
     assert np.abs(y - want).max() <= 2.0 ** -10 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("group", [32, 128])
+def test_rows_are_paired_only_for_the_kernel_that_reads_them(rng, group):
+    """Codes 4 bytes off the direct loads' alignment: the staged kernel runs, with
+    its bits, and the workspace for paired rows is left as it was."""
+    from local_kimi_amd import _lib
+    from local_kimi_amd.kernels import w4a16_dense_gemm
+
+    m, n, k = 40, 96, 256
+    x, (p, s) = random_bf16_bits(rng, (m, k)), _w4(rng, n, k, group)
+    dx, dp, ds = _dev(x), _dev(p), _dev(s)
+    moved = torch.empty(dp.numel() + 4, dtype=torch.uint8, device=DEV)
+    moved[4:].copy_(dp.view(-1))
+    ws = torch.full((_lib.query("lk_dense_gemm_workspace", m, n, k, group, 1, 0),), 0xA5,
+                    dtype=torch.uint8, device=DEV)
+    y = torch.empty((m, n), dtype=torch.bfloat16, device=DEV)
+    _lib.call("lk_w4a16_dense_gemm_ws", dx.data_ptr(), moved.data_ptr() + 4, ds.data_ptr(),
+              y.data_ptr(), m, n, k, group, ws.data_ptr(), ws.numel(),
+              torch.cuda.current_stream().cuda_stream)
+    assert torch.equal(y, w4a16_dense_gemm(dx, dp, ds))
+    assert bool((ws == 0xA5).all())
+
+
+def test_rows_beyond_the_pairing_run_staged(rng):
+    """2^27 row k-steps (34 GB of rows) at G = 32: more than one pairing launch
+    takes, and than the direct loads' offsets reach."""
+    from local_kimi_amd._lib import forced_path
+    from local_kimi_amd.kernels import w4a16_dense_gemm
+
+    m, n, k = 1 << 20, 32, 16384
+    if torch.cuda.mem_get_info()[0] < 60 << 30:
+        pytest.skip("needs 60 GB of device memory")
+    p, s = _w4(rng, n, k, 32)
+    x = torch.zeros((m, k), dtype=torch.bfloat16, device=DEV)
+    x[-80:] = torch.randn(80, k, device=DEV).to(torch.bfloat16)
+    x[:16] = x[-16:]
+    y = w4a16_dense_gemm(x, _dev(p), _dev(s))
+    with forced_path("dense_gemm", "lds"):
+        want = w4a16_dense_gemm(x[-80:].clone(), _dev(p), _dev(s))
+    assert torch.equal(y[-80:], want)
+    assert torch.equal(y[:16], want[-16:])
+    assert not bool(y[16:-80].any())
