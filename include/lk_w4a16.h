@@ -68,7 +68,10 @@ LK_API int lk_get_path(const char* knob);
 
 /* weight bf16 [N,K] -> packed [N,K/2], scales bf16 [N,K/G]; bit-exact with
  * the reference encoder (absmax/7 scale stored as bf16, codes rounded half
- * to even against the stored scale, clamped to [-7, 7]). */
+ * to even against the stored scale, clamped to [-7, 7]). Weights are meant to
+ * be finite; at every group width and address a NaN is left out of its group's
+ * absmax and gets the code -7, and an infinity makes its group's scale
+ * infinite (codes 0, and -7 for the infinity itself). */
 LK_API int lk_w4a16_quantise(const uint16_t* weight, uint8_t* packed, uint16_t* scales,
                       int64_t n, int64_t k, int64_t group_size, void* stream);
 

@@ -86,7 +86,9 @@ __device__ inline uint16_t group_scale(float absmax) {
 // residual step, the correctly rounded division inside the exponent range
 // below (v and s have 8 bits, so only an exact tie is within an ulp of a tie,
 // and its residual is exact); outside it the division itself.
-// nonfinite (null: not wanted) becomes 1 if any value is infinite or NaN.
+// A NaN is left out of its group's absmax, as the float maximum of the kernel
+// below leaves it out; nonfinite (null: not wanted) becomes 1 if any value is
+// infinite or NaN.
 template <int LANES>
 __global__ void __launch_bounds__(256)
 quantise_units_kernel(const uint16_t* __restrict__ w, uint32_t* __restrict__ packed,
@@ -99,12 +101,21 @@ quantise_units_kernel(const uint16_t* __restrict__ w, uint32_t* __restrict__ pac
   uint32_t big = 0;  // |v| as bits: ordered like the values, NaN above infinity
 #pragma unroll
   for (int i = 0; i < 4; ++i) big = max(big, max(d[i] & 0x7FFFu, (d[i] >> 16) & 0x7FFFu));
+  const uint32_t top = big;
+  if (big > 0x7F80u) {  // hardly ever: the maximum over the other values
+    big = 0;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t a = (d[i >> 1] >> (16 * (i & 1))) & 0x7FFFu;
+      big = max(big, a > 0x7F80u ? 0u : a);
+    }
+  }
   big = max(big, dpp_u32<kQuadXor1>(big));
   big = max(big, dpp_u32<kQuadXor2>(big));
   if constexpr (LANES >= 8) big = max(big, dpp_u32<kRowHalfMirror>(big));
   if constexpr (LANES >= 16) big = max(big, dpp_u32<kRowMirror>(big));
   if (!live) return;
-  if (nonfinite != nullptr && big >= 0x7F80u) *nonfinite = 1;
+  if (nonfinite != nullptr && top >= 0x7F80u) *nonfinite = 1;
   const uint16_t bits = group_scale(bf16_to_f32(static_cast<uint16_t>(big)));
   const float s = bf16_to_f32(bits);
   const float inv = 1.0f / s;

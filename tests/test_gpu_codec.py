@@ -64,3 +64,35 @@ def test_quantise_rejects_non_finite(rng, group, bad):
         quantise(w, group_size=group)
     w[4, 511] = 0.0
     quantise(w, group_size=group)
+
+
+@pytest.mark.parametrize("group", [32, 64, 128, 256])
+@pytest.mark.parametrize("shift", [0, 2])
+def test_c_quantiser_on_non_finite_weights(rng, group, shift):
+    """The C entry without a flag: a NaN (quiet or signalling) is left out of its
+    group's absmax and coded -7, an infinity makes the scale infinite; the other
+    groups are the oracle's. The same at every width and address."""
+    from local_kimi_amd import _lib
+
+    n, k = 6, 512
+    bits = f32_to_bf16_bits(rng.normal(0, 0.02, (n, k)).astype(np.float32))
+    bits[0, 3], bits[1, 300], bits[2, 511] = 0x7FC0, 0xFFC1, 0x7F81
+    bits[4, 17], bits[5, 200] = 0x7F80, 0xFF80
+    nan = (bits & 0x7FFF) > 0x7F80
+    inf = (bits & 0x7FFF) == 0x7F80
+    packed, scales = OW.quantise(np.where(nan | inf, 0, bits).astype(np.uint16), group)
+    codes = np.stack((packed & 15, packed >> 4), -1).reshape(n, k)
+    codes[nan | inf] = 9
+    wide = inf.reshape(n, -1, group).any(-1)
+    codes[np.repeat(wide, group, 1) & ~inf] = 0
+    scales[wide] = 0x7F80
+
+    flat = torch.empty(n * k + 8, dtype=torch.bfloat16, device=DEV)
+    w = flat[shift:shift + n * k]
+    w.copy_(from_bits(bits, DEV).view(-1))
+    got_p = torch.empty((n, k // 2), dtype=torch.uint8, device=DEV)
+    got_s = torch.empty((n, k // group), dtype=torch.bfloat16, device=DEV)
+    _lib.call("lk_w4a16_quantise", w.data_ptr(), got_p.data_ptr(), got_s.data_ptr(), n, k, group,
+              torch.cuda.current_stream().cuda_stream)
+    assert np.array_equal(to_bits(got_s), scales)
+    assert np.array_equal(got_p.cpu().numpy(), (codes[:, 0::2] | codes[:, 1::2] << 4).astype(np.uint8))
