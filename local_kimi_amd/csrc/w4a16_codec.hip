@@ -364,17 +364,20 @@ int lk_w4a16_quantise_checked(const uint16_t* weight, uint8_t* packed, uint16_t*
   LK_REQUIRE(n > 0, "output features must be positive");
   if (int rc = check_group(k, group_size)) return rc;
   hipStream_t s = as_stream(stream);
-  // 16-byte loads and dword stores where the operands allow them
-  const bool wide = (reinterpret_cast<uintptr_t>(weight) & 15) == 0 &&
-                    (reinterpret_cast<uintptr_t>(packed) & 3) == 0;
+  // 16-byte loads and dword stores where the operands allow them and the
+  // launch holds a thread per unit (a grid has fewer than 2^32 threads; the
+  // per-group kernel needs a fourth of them or less)
   const int64_t units = n * k / 8;
+  const bool wide = (reinterpret_cast<uintptr_t>(weight) & 15) == 0 &&
+                    (reinterpret_cast<uintptr_t>(packed) & 3) == 0 &&
+                    units <= (int64_t{1} << 32) - 256;
   auto* codes = reinterpret_cast<uint32_t*>(packed);
   const unsigned nb = blocks_for(units, 256);
-  if (wide && group_size == 32 && units < (1LL << 38))
+  if (wide && group_size == 32)
     quantise_units_kernel<4><<<nb, 256, 0, s>>>(weight, codes, scales, units, nonfinite);
-  else if (wide && group_size == 64 && units < (1LL << 38))
+  else if (wide && group_size == 64)
     quantise_units_kernel<8><<<nb, 256, 0, s>>>(weight, codes, scales, units, nonfinite);
-  else if (wide && group_size == 128 && units < (1LL << 38))
+  else if (wide && group_size == 128)
     quantise_units_kernel<16><<<nb, 256, 0, s>>>(weight, codes, scales, units, nonfinite);
   else
     quantise_kernel<<<blocks_for(n * (k / group_size), 256), 256, 0, s>>>(

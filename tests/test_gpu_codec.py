@@ -96,3 +96,26 @@ def test_c_quantiser_on_non_finite_weights(rng, group, shift):
               torch.cuda.current_stream().cuda_stream)
     assert np.array_equal(to_bits(got_s), scales)
     assert np.array_equal(got_p.cpu().numpy(), (codes[:, 0::2] | codes[:, 1::2] << 4).astype(np.uint8))
+
+
+def test_quantise_takes_more_weights_than_a_launch_has_threads(rng):
+    """2^35 weights: a thread per 8 of them is more than a launch holds, a thread
+    per group is not."""
+    from local_kimi_amd.quant import quantise
+
+    n, k = 1 << 21, 1 << 14
+    if torch.cuda.mem_get_info()[0] < 110 << 30:
+        pytest.skip("needs 110 GB of device memory")
+    some = f32_to_bf16_bits(rng.normal(0, 0.02, (3, k)).astype(np.float32))
+    w = torch.zeros((n, k), dtype=torch.bfloat16, device=DEV)
+    rows = [0, n // 2 + 1, n - 1]
+    for r, bits in zip(rows, some):
+        w[r] = from_bits(bits, DEV)
+    got = quantise(w)
+    packed, scales = OW.quantise(some, 32)
+    for i, r in enumerate(rows):
+        assert np.array_equal(got.packed[r].cpu().numpy(), packed[i])
+        assert np.array_equal(to_bits(got.scales[r]), scales[i])
+    assert not bool(got.packed[1:n // 2].any()) and bool((got.scales[1:n // 2] == 1).all())
+    del w, got
+    torch.cuda.empty_cache()
