@@ -2938,7 +2938,8 @@ int64_t dense_ws_bytes(bool mx, int64_t m, int64_t n, int64_t k, int64_t group, 
   const int64_t pairs = mx ? 0 : dense_pair_bytes(m, k, group);
   if (k % 128 != 0 || m < 1 || (!mx && pairs == 0)) return pairs;
   if (!tile_sizes(m, n, k)) return group == 128 ? pairs : 0;
-  return pairs + tile_gemm_split_bytes(mx, m, n, k, outputs);
+  return pairs + tile_gemm_split_bytes(mx ? kFmtMxBf16 : tile_format(kFmtW4A16, group), m, n, k,
+                                       outputs);
 }
 
 // Points the launch at the split sums when the workspace holds them (a

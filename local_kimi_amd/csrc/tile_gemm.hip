@@ -571,6 +571,15 @@ namespace {
 // their fp32 sums written and read at 6 TB/s; a split has to gain kTgGain.
 // 64 x 9216 -> 2304 at G = 32: 32 us in 8 runs against 70; 1000 rows 97
 // against 126; 200 x 2304 -> 9216 stays whole (31.4 against 34.2).
+// At G = 128 (one closing FMA per four MFMAs) 256-column blocks split too, into
+// at most kTgWideRuns runs of at least kTgWideRunSteps, where all of them are
+// resident: estimated
+// at 1.55 of a 128-column block's step, 0.55 of that for each further one, and
+// taken where that is kTgWideGain of the other estimate. 9216 -> 2304, us, the
+// 8-wave kernel before, 128 columns, these: 1100 rows 87, 93, 74; 1200 rows
+// 89, 96, 90; 1400 rows 92, 99, 94; 2048 x 8192 -> 1024 74 against 61. Of 184
+// products of 16 to 4096 rows it changed 20: 0.79 to 1.05 of the time. At
+// groups of 32 and 64 the same estimate lost up to 16 % on some.
 constexpr double kTgWideSlots = 512.0;
 constexpr int64_t kTgRunSteps = 4;
 // shorter products stay whole (little to gain, and their outputs stay the
@@ -578,26 +587,34 @@ constexpr int64_t kTgRunSteps = 4;
 constexpr int64_t kTgSplitSteps = 24;
 constexpr int64_t kTgMaxRuns = 16;
 constexpr double kTgGain = 6.0;
+constexpr int64_t kTgWideRunSteps = 16;
+constexpr int64_t kTgWideRuns = 4;  // eight lost up to 6 % at 16384 -> 512
+constexpr double kTgWideGain = 0.95;
 
 struct DensePlan {
   bool narrow;
   int64_t steps, runs;  // k-steps per run, runs
 };
 
-DensePlan dense_plan(bool mx, int64_t m, int64_t n, int64_t k, int64_t outputs, bool may_split) {
+DensePlan dense_plan(int fmt, int64_t m, int64_t n, int64_t k, int64_t outputs, bool may_split) {
   const int64_t tiles = (m + kTileRows - 1) / kTileRows, ksteps = k / 128;
   const double r = static_cast<double>(tiles * ((n + 255) / 256) * outputs) / kTgWideSlots;
   const double part = r - static_cast<double>(static_cast<int64_t>(r));
+  const bool mx = !fmt_is_w4(fmt);
   const bool wide = r >= 3.0 || (r >= 0.8 && (part == 0.0 || part >= 0.4));
   DensePlan p{!wide, ksteps, 1};
   if (!p.narrow || !may_split || ksteps < kTgSplitSteps) return p;
   const double blocks = static_cast<double>(tiles * ((n + 127) / 128) * outputs);
+  const double wide_blocks = static_cast<double>(tiles * ((n + 255) / 256) * outputs);
   const double subtiles = static_cast<double>((std::min<int64_t>(m, kTileRows) + 15) / 16);
   const double step = mx ? 0.35 + 0.1 * subtiles : 0.65 + 0.17 * subtiles;
-  auto estimate = [&](int64_t steps, int64_t runs) {
-    const double per_cu = std::max(1.0, blocks * runs / 256.0);
+  auto estimate_of = [&](double count, double one, double further, int64_t steps, int64_t runs) {
+    const double per_cu = std::max(1.0, count * runs / 256.0);
     const double sums = runs > 1 ? 5.0 + 8e-6 / 6.0 * runs * m * n * outputs : 0.0;
-    return steps * step * (1.0 + 0.6 * (per_cu - 1.0)) + sums;
+    return steps * one * (1.0 + further * (per_cu - 1.0)) + sums;
+  };
+  auto estimate = [&](int64_t steps, int64_t runs) {
+    return estimate_of(blocks, step, 0.6, steps, runs);
   };
   double best = estimate(ksteps, 1) - kTgGain;
   for (int64_t want = 2; want <= std::min(ksteps / kTgRunSteps, kTgMaxRuns); ++want) {
@@ -609,13 +626,24 @@ DensePlan dense_plan(bool mx, int64_t m, int64_t n, int64_t k, int64_t outputs, 
       p.runs = runs;
     }
   }
+  if (fmt != kFmtW4A16) return p;
+  double most = best * kTgWideGain;
+  for (int64_t want = 2; want <= std::min(ksteps / kTgWideRunSteps, kTgWideRuns); ++want) {
+    const int64_t steps = (ksteps + want - 1) / want, runs = (ksteps + steps - 1) / steps;
+    if (wide_blocks * runs > kTgWideSlots) break;
+    const double t = estimate_of(wide_blocks, 1.55 * step, 0.55, steps, runs);
+    if (t < most) {
+      most = t;
+      p = {false, steps, runs};
+    }
+  }
   return p;
 }
 
 }  // namespace
 
-int64_t tile_gemm_split_bytes(bool mx, int64_t m, int64_t n, int64_t k, int64_t outputs) {
-  const DensePlan p = dense_plan(mx, m, n, k, outputs, true);
+int64_t tile_gemm_split_bytes(int fmt, int64_t m, int64_t n, int64_t k, int64_t outputs) {
+  const DensePlan p = dense_plan(fmt, m, n, k, outputs, true);
   return p.runs > 1 ? p.runs * m * n * outputs * 4 : 0;
 }
 
@@ -623,7 +651,7 @@ int tile_gemm_launch(int fmt, int mats, GemmArgs g, Mode mode, int64_t tiles, hi
                      const char* what) {
   const bool dense = mode == Mode::Dense;
   const bool split = dense && g.part != nullptr;
-  const DensePlan plan = dense ? dense_plan(!fmt_is_w4(fmt), g.dense_rows, g.n, g.k, g.outputs, split)
+  const DensePlan plan = dense ? dense_plan(fmt, g.dense_rows, g.n, g.k, g.outputs, split)
                                : DensePlan{false, g.k / 128, 1};
   if (plan.runs == 1) g.part = nullptr;
   g.split_steps = static_cast<int>(plan.steps);

@@ -16,7 +16,7 @@ int tile_gemm_launch(int fmt, int mats, GemmArgs g, Mode mode, int64_t tiles, hi
                      const char* what);
 
 // Bytes of the fp32 sums of a dense [m, k] x [k, outputs * n] product that is
-// worth splitting over k; 0 where it is not.
-int64_t tile_gemm_split_bytes(bool mx, int64_t m, int64_t n, int64_t k, int64_t outputs);
+// worth splitting over k in weight format kFmt*; 0 where it is not.
+int64_t tile_gemm_split_bytes(int fmt, int64_t m, int64_t n, int64_t k, int64_t outputs);
 
 }  // namespace lk

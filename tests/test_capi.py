@@ -103,6 +103,19 @@ def test_dense_workspace_covers_only_what_the_prefill_gemm_takes(lib):
     assert lib.lk_dense_gemm_workspace(1 << 20, 256, 1024, 32, 1, 0) > (1 << 31)
 
 
+def test_dense_split_runs_of_256_column_blocks(lib):
+    """9216 -> 2304 and 8192 -> 1024 at G = 128: too few 256-column blocks for the
+    chip, taken in two to four runs of k (fp32 sums of every run behind the
+    paired rows); at groups of 32 the 128-column blocks' runs stay."""
+    def runs(m, n, k, group):
+        pairs = 2 * m * k + 4 * m * (k // 128) * (1 if group == 128 else 4)
+        return (lib.lk_dense_gemm_workspace(m, n, k, group, 1, 0) - pairs) // (4 * m * n)
+
+    assert [runs(m, 2304, 9216, 128) for m in (768, 1024, 1280, 1600)] == [4, 3, 2, 2]
+    assert [runs(m, 1024, 8192, 128) for m in (2048, 2560, 4096)] == [4, 3, 2]
+    assert [runs(m, 2304, 9216, 32) for m in (1280, 1600)] == [3, 0]
+
+
 def test_grouped_router_argument_errors(lib):
     # (logits, bias, idx, w, tokens, experts, top_k, groups, topk_group, scale, renorm, stream)
     with pytest.raises(RuntimeError, match="divisible"):

@@ -222,3 +222,15 @@ def test_rows_beyond_the_pairing_run_staged(rng):
     assert torch.equal(y[-80:], want)
     assert torch.equal(y[:16], want[-16:])
     assert not bool(y[16:-80].any())
+
+
+@pytest.mark.parametrize("m,n,k", [(700, 2304, 9216), (1600, 1001, 8192)])
+def test_dense_split_of_256_column_blocks_matches_oracle(rng, m, n, k):
+    """256-column blocks in four runs of k (G = 128): a ragged last row tile, odd
+    widths; the oracle on rows of every kind of tile."""
+    from local_kimi_amd.kernels import w4a16_dense_gemm
+
+    x, (p, s) = random_bf16_bits(rng, (m, k)), _w4(rng, n, k, 128)
+    y = to_bits(w4a16_dense_gemm(_dev(x), _dev(p), _dev(s)))
+    rows = np.unique(np.concatenate(([0, 15, 16, 63, 64, m - 65, m - 1], rng.integers(0, m, 8))))
+    assert_close_bf16(y[rows], OW.dense(x[rows], p, s, 128), what=f"wide split {m}x{n}x{k}")
