@@ -52,6 +52,16 @@ struct TgStage {
   static constexpr int kU4 = kScaleAt + W * kScaleU4;
 };
 
+// Codes of output matrix i, chosen by masks: of pick3's branches on these
+// pointers the compiler made a copy of all three in scratch memory, stored by
+// every block and read back by index (32 bytes a lane of every launch).
+__device__ inline const uint8_t* codes_of(const GemmArgs& g, int i) {
+  const uint64_t one = -static_cast<uint64_t>(i == 1), two = -static_cast<uint64_t>(i == 2);
+  return reinterpret_cast<const uint8_t*>(
+      (reinterpret_cast<uint64_t>(g.wp[0]) & ~(one | two)) |
+      (reinterpret_cast<uint64_t>(g.wp[1]) & one) | (reinterpret_cast<uint64_t>(g.wp[2]) & two));
+}
+
 template <int TILES, int FMT, int MATS, int MT, bool GATHER, bool SCATTER, bool DENSE>
 __device__ __forceinline__ void tg_tile(const GemmArgs& g, uint4* const lds, const int expert,
                                         const int row0, const int rows, const int cb,
@@ -115,7 +125,7 @@ __device__ __forceinline__ void tg_tile(const GemmArgs& g, uint4* const lds, con
   u32x4_t rs_w[MATS], rs_s[MATS];
 #pragma unroll
   for (int mi = 0; mi < MATS; ++mi) {
-    rs_w[mi] = buffer_rsrc(pick3(g.wp, osel + mi) + expert * g.wstride, N * rowb);
+    rs_w[mi] = buffer_rsrc(codes_of(g, osel + mi) + expert * g.wstride, N * rowb);
     // (an odd count of scales: the last dword's valid half must not read as zero)
     rs_s[mi] = buffer_rsrc(static_cast<const uint8_t*>(pick3(g.ws, osel + mi)) +
                                expert * g.sstride * kSb,

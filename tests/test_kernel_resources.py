@@ -75,3 +75,10 @@ def test_persistent_gemms_hold_their_ring_in_registers(kernels):
             continue
         assert k[".vgpr_spill_count"] <= 16, (k[".name"], k[".vgpr_spill_count"])
     assert seen > 50
+
+
+def test_prefill_gemms_use_no_scratch_memory(kernels):
+    sizes = {k[".name"]: k[".private_segment_fixed_size"] for k in kernels
+             if _template_args(k[".name"], "tile_gemm_kernel") is not None}
+    assert len(sizes) >= 18
+    assert not {name: size for name, size in sizes.items() if size}
