@@ -234,3 +234,38 @@ def test_dense_split_of_256_column_blocks_matches_oracle(rng, m, n, k):
     y = to_bits(w4a16_dense_gemm(_dev(x), _dev(p), _dev(s)))
     rows = np.unique(np.concatenate(([0, 15, 16, 63, 64, m - 65, m - 1], rng.integers(0, m, 8))))
     assert_close_bf16(y[rows], OW.dense(x[rows], p, s, 128), what=f"wide split {m}x{n}x{k}")
+
+
+@pytest.mark.parametrize("k", [128, 384])
+@pytest.mark.parametrize("n", [5000, 5001])
+@pytest.mark.parametrize("weights", ["g32", "g64", "g128", "bf16", "f16"])
+def test_dense_256_column_blocks(rng, weights, n, k):
+    """Enough blocks (21 x 20) for 256 columns each: a ragged last row tile and
+    last column block, values one by one (n = 5001), an odd number of k-steps,
+    the even split over the XCDs. W4A16 against the LDS-staged kernel's bits,
+    and everything against the oracle on sampled rows."""
+    from local_kimi_amd._lib import forced_path
+    from local_kimi_amd.kernels import mxfp4_gemm, w4a16_dense_gemm
+
+    m = 1301
+    rows = np.array([0, 15, 16, 63, 64, 700, 1279, 1280, 1300])
+    if weights[0] == "g":
+        group = int(weights[1:])
+        x, (p, s) = random_bf16_bits(rng, (m, k)), _w4(rng, n, k, group)
+        args = (_dev(x), _dev(p), _dev(s))
+        y = w4a16_dense_gemm(*args)
+        with forced_path("dense_gemm", "lds"):
+            assert torch.equal(y, w4a16_dense_gemm(*args))
+        assert_close_bf16(to_bits(y)[rows], OW.dense(x[rows], p, s, group), what=f"{weights} {n} {k}")
+        return
+    p, s = _mx(rng, n, k)
+    if weights == "bf16":
+        x = random_bf16_bits(rng, (m, k))
+        y = mxfp4_gemm(_dev(x), _dev(p), _dev(s))
+        assert_close_bf16(to_bits(y)[rows], X.linear(x[rows], p, s), what=f"mxfp4 {n} {k}")
+    else:
+        x = rng.normal(0, 1, (m, k)).astype(np.float16)
+        y = mxfp4_gemm(torch.from_numpy(x).to(DEV), _dev(p), _dev(s)).float().cpu().numpy()[rows]
+        want = x[rows].astype(np.float64) @ X.dequantize(p, s).astype(np.float64).T
+        # one rounding to fp16 (2^-11) of an fp32 sum
+        assert np.abs(y - want).max() <= 2.0 ** -10 * np.abs(want).max()
