@@ -279,7 +279,11 @@ LK_API int lk_w4a16_fused_qkv(const uint16_t* x, const uint8_t* q_packed,
  * With lk_dense_gemm_workspace(m, n, k, group, outputs, mxfp4) bytes (outputs:
  * 3 for the fused QKV, else 1; mxfp4 != 0: lk_mxfp4_gemm_ws, group 32; never
  * less than the query above) groups of 32 and 64 take that GEMM too, and a
- * product too small to fill the GPU is split over k. */
+ * product too small to fill the GPU is split over k: from k = 3072 the number
+ * of runs follows m and n, so a row's last bf16 bit can differ between calls
+ * of different m. Where the number of scales (n * k / group) is odd, that GEMM
+ * reads the dword that holds the last one whole, 2 bytes past the operand (an
+ * aligned dword; the other half is not used). */
 LK_API int64_t lk_w4a16_dense_gemm_workspace(int64_t m, int64_t k, int64_t group_size);
 LK_API int64_t lk_dense_gemm_workspace(int64_t m, int64_t n, int64_t k, int64_t group_size,
                                        int64_t outputs, int mxfp4);

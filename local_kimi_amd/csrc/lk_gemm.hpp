@@ -110,7 +110,7 @@ __device__ inline bf16x8_t unpack_q8(uint32_t w) {
 // half-wave swaps and two row swaps. The four dwords loaded apart (and four
 // 2-byte scales) are eight loads a k-step instead of two: at 16 tokens of the
 // Kimi-Linear layer with G = 32 they held the block to 1.0 TB/s, 416 us with
-// its norms and router, against 147 us on the persistent kernel in this form.
+// its norms and router, against 118 us on the persistent kernel in this form.
 __device__ inline void transpose4(uint32_t (&w)[4]) {
   auto half = [](uint32_t& a, uint32_t& b) {
     const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);

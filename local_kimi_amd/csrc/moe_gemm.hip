@@ -1375,17 +1375,6 @@ __device__ inline void ps_stage_store(uint4* afrag, float* offs, int frag, int c
   }
 }
 
-// Two consecutive 128-wide k-steps (2q, 2q + 1) of a lane's weights for the
-// persistent kernel: per matrix and column tile, the two 16-byte code loads
-// are issued back to back (they are the two halves of one 128-byte line of
-// the weight row, so the line is fetched once: requested apart, each half
-// costs a fetch of its own), and one scale load serves both steps (W4A16
-// G = 128: the bf16 pair, low half = step 2q; G = 64 and 32: the pair's two
-// and four dwords of bf16, one per lane block, spread by ps_scale_dwords where
-// they are used: held whole they are up to 12 registers of ring more, which
-// spilled; MXFP4: eight E8M0 bytes, four per step). Whole-dword scale loads keep the ring free of narrow loads, whose
-// zero-extension the compiler otherwise places at the loop latch, where it
-// waits for every load in flight.
 // Step h's scale dwords (G = 32: dwords 2 h and 2 h + 1 of the pair's four, in
 // lane blocks 0 .. 3; G = 64: dword h of two, in lane blocks 0, 1, 0, 1) in
 // every lane.
@@ -1403,6 +1392,17 @@ __device__ inline void ps_scale_dwords(uint32_t s, int h, uint32_t (&d)[CHAIN ==
   }
 }
 
+// Two consecutive 128-wide k-steps (2q, 2q + 1) of a lane's weights for the
+// persistent kernel: per matrix and column tile, the two 16-byte code loads
+// are issued back to back (they are the two halves of one 128-byte line of
+// the weight row, so the line is fetched once: requested apart, each half
+// costs a fetch of its own), and one scale load serves both steps (W4A16
+// G = 128: the bf16 pair, low half = step 2q; G = 64 and 32: the pair's two
+// and four dwords of bf16, one per lane block, spread by ps_scale_dwords where
+// they are used: held whole they are up to 12 registers of ring more, which
+// spilled; MXFP4: eight E8M0 bytes, four per step). Whole-dword scale loads
+// keep the ring free of narrow loads, whose zero-extension the compiler
+// otherwise places at the loop latch, where it waits for every load in flight.
 template <int FMT, int MATS, int NT>
 struct PsPair {
   static constexpr int kSw = fmt_is_w4(FMT) ? 1 : 2;  // scale dwords per lane and pair
@@ -2838,10 +2838,18 @@ int stream_fmt(bool mx, const GemmArgs& g, Mode mode, int64_t tiles, int mt, hip
   return stream_launch<kFmtW4A16, MATS>(g, mode, tiles, mt, s, what);
 }
 
-// Expert-major calls use the streaming kernel: 16-row tiles up to
-// kStreamSmallEntries token-routes (decode batches, few rows per expert),
-// 64-row tiles above (prefill). The path knob moe_gemm=lds selects the
-// LDS-staged kernel instead, moe_gemm=stream16|stream64 forces a tile height.
+// Expert-major calls take 16-row tiles up to kStreamSmallEntries token-routes
+// (decode batches, few rows per expert: the persistent kernel), the prefill
+// GEMM's 64-row tiles above. The path knob moe_gemm=lds selects the LDS-staged
+// kernel instead, moe_gemm=stream16|stream64 forces a tile height. Where the
+// two heights cross, in every format, is at about 16 rows per expert: 128
+// experts of 2304 x 1536 (us, 16 : 64 rows) at 1800 and 2300 routes G = 64
+// 211 : 230 and 252 : 240, G = 128 201 : 201 and 230 : 212, MXFP4 208 : 213 and
+// 247 : 221; so with 256 experts the line is early (Kimi-Linear layer at 2304
+// routes G = 32 282 : 339, G = 128 233 : 247, at 4608 385 : 370 and 332 : 285)
+// and with 64 late (2048 x 1024 at 1440 G = 128 101 : 89). G = 32 with both
+// matrices in a unit that spills (intermediates above 1024 at k = 2304) is
+// faster on 64 rows from 432 routes on (420 : 245).
 constexpr int64_t kStreamSmallEntries = 2048;
 
 // Which MFMA form the MXFP4 expert GEMMs take: bf16 MFMA on weights decoded

@@ -1,6 +1,6 @@
-// Prefill GEMM: tiles of at most 64 rows x 256 weight columns (128 of gate and
-// 128 of up), one block of 4 waves each, two blocks per CU; x 128 columns
-// where that would leave the chip idle.
+// Prefill GEMM: tiles of at most 64 rows (dense; 80 in the expert-major merged
+// list) x 256 weight columns (128 of gate and 128 of up), one block of 4 waves
+// each, two blocks per CU; x 128 columns where that would leave the chip idle.
 //
 // What bounds it is the vector L1: a load whose neighbouring lanes read
 // different weight rows (an MFMA operand's own layout: lane = column) costs
@@ -9,15 +9,17 @@
 // global -> LDS loads whose lanes run along k (4 lanes of 16 bytes per weight
 // row and k-step), and the operand layout is made by the LDS read, of which
 // there is plenty: an A fragment feeds TILES MFMAs.
-// Measured (us, before: the 8-wave kernels with weights loaded straight into
-// registers): 2048 x 2304 x 12288 at G = 128 156 -> 123 (940 TFLOP/s, MFMA 44 %
-// and VALU 37 % of the SIMD cycles at 2.04 GHz), 1500 x 4096 x 2304 at G = 32
-// 153 -> 63, 333 x 2304 x 9216 MXFP4 on fp16 rows 111 -> 19, the MoE block of
-// 2048 tokens at G = 128 495 -> 430, of 777 tokens at G = 32 (with its router)
-// 1246 -> 408. At groups of 32 the VALU bounds it (one FMA per output and MFMA);
-// with few rows per expert the weights' stream from HBM does.
-// A k-step is 128 of k. The loads of step s + kStages - 1 are issued while
-// step s computes; a wait and one barrier a step publish the next stage.
+// Measured in turn (us a call, before: the 8-wave kernels with weights loaded
+// straight into registers): 2048 x 2304 x 12288 at G = 128 141 -> 121 (960
+// TFLOP/s, MFMA 44 % and VALU 37 % of the SIMD cycles at 2.04 GHz), 1500 x 4096
+// x 2304 at G = 32 152 -> 63, 333 x 2304 x 9216 MXFP4 on fp16 rows 111 -> 19, the
+// MoE block of 2048 tokens at G = 128 466 -> 428, of 777 tokens at G = 32 (with
+// its router) 1239 -> 409. At groups of 32 no unit is full (1500 rows: VALU
+// 30 %, LDS 29 %, MFMA 17 % of the cycles, 1.3 waves per SIMD; 777 tokens: VALU
+// 34 %, MFMA 13 %, the banks read once at 2.4 TB/s): each k-step waits for the
+// loads of the next, with few waves to fill the time.
+// A k-step is 128 of k. The loads of step s + 1 are issued while step s
+// computes; a wait and one barrier a step publish the next stage.
 
 #include <algorithm>
 
@@ -73,7 +75,6 @@ __device__ __forceinline__ void tg_tile(const GemmArgs& g, uint4* const lds, con
   constexpr int kBN = W * NT * 16;
   typedef TgStage<TILES, FMT, tg_rows(DENSE)> St;
   constexpr int kRowLoads = MT;  // 4-row loads per wave and k-step
-  constexpr int kLoads = kRowLoads + (kW4 ? 1 : 0) + TILES + MATS * St::kScaleDwords;  // per wave and k-step
   const int64_t N = g.n, K = g.k;
   // this block's k-steps: all, or the blockIdx.y-th run of a split product
   const int all_steps = static_cast<int>(K >> 7);
@@ -126,7 +127,8 @@ __device__ __forceinline__ void tg_tile(const GemmArgs& g, uint4* const lds, con
 #pragma unroll
   for (int mi = 0; mi < MATS; ++mi) {
     rs_w[mi] = buffer_rsrc(codes_of(g, osel + mi) + expert * g.wstride, N * rowb);
-    // (an odd count of scales: the last dword's valid half must not read as zero)
+    // (an odd count of scales: the last dword's valid half must not read as
+    // zero, so that dword is read whole, 2 bytes past the tensor)
     rs_s[mi] = buffer_rsrc(static_cast<const uint8_t*>(pick3(g.ws, osel + mi)) +
                                expert * g.sstride * kSb,
                            (N * spr * kSb + 3) & ~int64_t{3});
@@ -144,8 +146,7 @@ __device__ __forceinline__ void tg_tile(const GemmArgs& g, uint4* const lds, con
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_offset(lds));
   auto load_step = [&](int step_, int stage) {
     const int local = __builtin_amdgcn_readfirstlane(step_);
-    // past the last k-step: descriptors of no bytes (zeros, no traffic), so
-    // every path has the same loads in flight
+    // past the last k-step: descriptors of no bytes (zeros, no traffic)
     const bool live = local < ksteps;
     const int step = first_step + local;
     auto only = [&](u32x4_t r) {
@@ -308,21 +309,18 @@ __device__ __forceinline__ void tg_tile(const GemmArgs& g, uint4* const lds, con
     }
   };
 
-  // the stream: step s computes from stage s % kStages while the loads of the
-  // steps up to s + kStages - 1 are in flight. The wait leaves the loads of
-  // the steps after s + 1 in flight, so this wave's part of step s + 1 has
-  // landed; the barrier publishes it and retires stage s % kStages.
-  constexpr int kAhead = kTgStages - 1;
-#pragma unroll
-  for (int j = 0; j < kAhead; ++j) load_step(j, j);
-  wait_vmcnt<(kAhead - 1) * kLoads>();
+  // the stream: step s computes from stage s % 2 while the loads of step s + 1
+  // are in flight. The wait is for all of them, so this wave's part of step
+  // s + 1 has landed; the barrier publishes it and retires stage s % 2.
+  load_step(0, 0);
+  wait_vmcnt<0>();
   __syncthreads();
   auto one = [&](int s, int stage) {
-    load_step(s + kAhead, (stage + kAhead) % kTgStages);
+    load_step(s + 1, stage ^ 1);
     __builtin_amdgcn_sched_barrier(0);
     compute(s, stage);
     __builtin_amdgcn_sched_barrier(0);
-    wait_vmcnt<(kAhead - 1) * kLoads>();
+    wait_vmcnt<0>();
     __syncthreads();
   };
   for (int s = 0;;) {
@@ -466,7 +464,9 @@ __global__ void __launch_bounds__(W * kWave, TILES == 4 ? 2 : 3) tile_gemm_kerne
     row0 = __builtin_amdgcn_readfirstlane(d.y);
     rows = __builtin_amdgcn_readfirstlane(d.z);
   }
-  if (expert < 0) {  // routes outside the bank produce zero rows
+  // routes outside the bank produce zero rows (the MoE block routes itself and
+  // has none; a guard against reading in front of the bank)
+  if (expert < 0) {
     uint16_t* const out = pick3(g.out, osel);
     for (int i = threadIdx.x; i < rows * kBN; i += W * kWave) {
       const int m = i / kBN;

@@ -1,4 +1,4 @@
-// The 64-row prefill GEMM (tile_gemm.hip).
+// The prefill GEMM (tile_gemm.hip): tiles of 64 rows, 80 in the merged list.
 
 #pragma once
 
@@ -6,8 +6,8 @@
 
 namespace lk {
 
-// Launches the prefill GEMM over `tiles` row tiles of at most 64 rows (an
-// upper bound in schedule modes) for a weight format kFmt*: Gather (two
+// Launches the prefill GEMM over `tiles` row tiles (an upper bound in schedule
+// modes) for a weight format kFmt*: Gather (two
 // matrices), Scatter or Dense (one). The caller has checked the operands and
 // set a_pair / a_neg (W4A16) and a_rows; with g.part (device memory of
 // tile_gemm_split_bytes) a dense product too small to fill the chip runs in
