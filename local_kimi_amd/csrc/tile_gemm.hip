@@ -14,10 +14,10 @@
 // TFLOP/s, MFMA 44 % and VALU 37 % of the SIMD cycles at 2.04 GHz), 1500 x 4096
 // x 2304 at G = 32 152 -> 63, 333 x 2304 x 9216 MXFP4 on fp16 rows 111 -> 19, the
 // MoE block of 2048 tokens at G = 128 466 -> 428, of 777 tokens at G = 32 (with
-// its router) 1239 -> 409. At groups of 32 no unit is full (1500 rows: VALU
-// 30 %, LDS 29 %, MFMA 17 % of the cycles, 1.3 waves per SIMD; 777 tokens: VALU
-// 34 %, MFMA 13 %, the banks read once at 2.4 TB/s): each k-step waits for the
-// loads of the next, with few waves to fill the time.
+// its router) 1239 -> 409. At groups of 32 no unit is full at 1500 rows (VALU
+// 30 %, LDS 29 %, MFMA 17 % of the cycles, 1.3 waves per SIMD): each k-step waits
+// for the loads of the next, with few waves to fill the time. At 777 tokens the
+// gate/up launch fetches 1.8 times its banks, at 4.7 TB/s.
 // A k-step is 128 of k. The loads of step s + 1 are issued while step s
 // computes; a wait and one barrier a step publish the next stage.
 
