@@ -183,24 +183,77 @@ def test_fused_qkv_and_mxfp4_split_over_k_match_oracle(rng):
 
 @pytest.mark.parametrize("group", [32, 128])
 def test_rows_are_paired_only_for_the_kernel_that_reads_them(rng, group):
-    """Codes 4 bytes off the direct loads' alignment: the staged kernel runs, with
-    its bits, and the workspace for paired rows is left as it was."""
+    """Scales off the direct loads' dwords: the staged kernel runs, with its bits,
+    and the workspace for paired rows is left as it was."""
     from local_kimi_amd import _lib
     from local_kimi_amd.kernels import w4a16_dense_gemm
 
     m, n, k = 40, 96, 256
     x, (p, s) = random_bf16_bits(rng, (m, k)), _w4(rng, n, k, group)
     dx, dp, ds = _dev(x), _dev(p), _dev(s)
-    moved = torch.empty(dp.numel() + 4, dtype=torch.uint8, device=DEV)
-    moved[4:].copy_(dp.view(-1))
+    moved = torch.empty(ds.numel() + 1, dtype=torch.bfloat16, device=DEV)
+    moved[1:].copy_(ds.view(-1))
     ws = torch.full((_lib.query("lk_dense_gemm_workspace", m, n, k, group, 1, 0),), 0xA5,
                     dtype=torch.uint8, device=DEV)
     y = torch.empty((m, n), dtype=torch.bfloat16, device=DEV)
-    _lib.call("lk_w4a16_dense_gemm_ws", dx.data_ptr(), moved.data_ptr() + 4, ds.data_ptr(),
+    _lib.call("lk_w4a16_dense_gemm_ws", dx.data_ptr(), dp.data_ptr(), moved.data_ptr() + 2,
               y.data_ptr(), m, n, k, group, ws.data_ptr(), ws.numel(),
               torch.cuda.current_stream().cuda_stream)
     assert torch.equal(y, w4a16_dense_gemm(dx, dp, ds))
     assert bool((ws == 0xA5).all())
+
+
+def _shifted(t, by):
+    """A copy of t, `by` bytes off the allocator's alignment."""
+    buf = torch.empty(t.numel() * t.element_size() + 16, dtype=torch.uint8, device=DEV)
+    return buf[by:by + t.numel() * t.element_size()].view(t.dtype).view(t.shape).copy_(t)
+
+
+@pytest.mark.parametrize("by", [4, 8, 12])
+@pytest.mark.parametrize("weights", ["g32", "g64", "g128", "mxfp4"])
+def test_operands_on_any_dword_keep_the_prefill_gemm(rng, weights, by):
+    """Codes, scales and rows on a dword that no 16-byte line starts at: the same
+    bits, from the same kernel (a dense W4A16 call writes its workspace)."""
+    from local_kimi_amd import _lib
+    from local_kimi_amd._lib import forced_path
+    from local_kimi_amd.kernels import mxfp4_gemm, mxfp4_moe_block, w4a16_moe_forward
+
+    m, n, k = 100, 264, 640
+    stream = torch.cuda.current_stream().cuda_stream
+    if weights == "mxfp4":
+        x, (p, s) = random_bf16_bits(rng, (m, k)), _mx(rng, n, k)
+        dx, dp, ds = _dev(x), _dev(p), _dev(s)
+        assert torch.equal(mxfp4_gemm(*(_shifted(t, by) for t in (dx, dp, ds))), mxfp4_gemm(dx, dp, ds))
+        group, one, block = 32, _mx, mxfp4_moe_block
+    else:
+        group = int(weights[1:])
+        x, (p, s) = random_bf16_bits(rng, (m, k)), _w4(rng, n, k, group)
+        dx, dp, ds = _dev(x), _dev(p), _dev(s)
+        out = []
+        for args in ((dx, dp, ds), tuple(_shifted(t, by) for t in (dx, dp, ds))):
+            ws = torch.full((_lib.query("lk_dense_gemm_workspace", m, n, k, group, 1, 0),), 0xA5,
+                            dtype=torch.uint8, device=DEV)
+            y = torch.empty((m, n), dtype=torch.bfloat16, device=DEV)
+            _lib.call("lk_w4a16_dense_gemm_ws", *(t.data_ptr() for t in args), y.data_ptr(), m, n, k,
+                      group, ws.data_ptr(), ws.numel(), stream)
+            assert not bool((ws == 0xA5).all()), "not the prefill GEMM"
+            out.append(y)
+        assert torch.equal(*out)
+        one, block = (lambda r, nn, kk: _w4(r, nn, kk, group)), w4a16_moe_forward
+
+    e_routed, top_k, h, inter, tokens = 7, 2, 384, 256, 150
+
+    def bank(nn, kk):
+        enc = [one(rng, nn, kk) for _ in range(e_routed + 1)]
+        return _dev(np.stack([c for c, _ in enc])), _dev(np.stack([c for _, c in enc]))
+
+    banks = (*bank(inter, h), *bank(inter, h), *bank(h, inter))
+    hx = _dev(random_bf16_bits(rng, (tokens, h)))
+    logits = _dev(rng.normal(0, 1, (tokens, e_routed)).astype(np.float32))
+    with forced_path("moe_gemm", "stream64"):
+        y0 = block(hx, logits, None, *banks, top_k, 2.446)[0]
+        y1 = block(_shifted(hx, by), logits, None, *(_shifted(b, by) for b in banks), top_k, 2.446)[0]
+    assert torch.equal(y0, y1)
 
 
 def test_rows_beyond_the_pairing_run_staged(rng):
