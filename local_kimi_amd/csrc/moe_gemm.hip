@@ -2770,17 +2770,14 @@ int tile_format(int fmt, int64_t group) {
   return group == 128 ? kFmtW4A16 : group == 64 ? kFmtW4G64 : group == 32 ? kFmtW4G32 : -1;
 }
 
-// Whether the operands lie as the prefill GEMM takes them: what it stores in
-// 16-byte chunks on 16 bytes, what it loads directly (codes, scales, MXFP4
-// rows) on dwords, which is all that buffer loads ask for. (Banks 4 bytes off a 16-byte line on
-// the staged kernels: 2048 tokens of the Kimi-Linear layer at G = 128 690 us,
-// 548 on the 8-wave kernel before this one.)
-bool tile_aligned(std::initializer_list<const void*> stored,
-                  std::initializer_list<const void*> loaded) {
-  uintptr_t st = 0, ld = 0;
-  for (const void* p : stored) st |= reinterpret_cast<uintptr_t>(p);
-  for (const void* p : loaded) ld |= reinterpret_cast<uintptr_t>(p);
-  return (st & 15) == 0 && (ld & 3) == 0;
+// Whether the operands lie as the prefill GEMM takes them: on dwords, which is
+// all that its direct loads and its 16-byte stores ask for. (Banks 4 bytes off
+// a 16-byte line on the staged kernels: 2048 tokens of the Kimi-Linear layer
+// at G = 128 691 us, 548 on the 8-wave kernel before this one, 504 here.)
+bool tile_aligned(std::initializer_list<const void*> operands) {
+  uintptr_t any = 0;
+  for (const void* p : operands) any |= reinterpret_cast<uintptr_t>(p);
+  return (any & 3) == 0;
 }
 
 // Whether a dense product's rows and codes lie within the prefill GEMM's 32-bit
@@ -2798,9 +2795,8 @@ bool tile_fits(const GemmArgs& g, int fmt) {
   if (path_choice(kKnobDenseGemm) == 1 || tf < 0 || g.k % 128 != 0 || g.a_rows <= 0) return false;
   if (!tile_sizes(g.a_rows, g.n, g.k)) return false;
   if (fmt_is_w4(tf) && !(g.a_pair && g.a_neg)) return false;
-  return tile_aligned({fmt_is_w4(tf) ? g.a_pair : nullptr, g.out[0], g.out[1], g.out[2]},
-                      {fmt_is_w4(tf) ? nullptr : g.a, g.wp[0], g.wp[1], g.wp[2], g.ws[0], g.ws[1],
-                       g.ws[2]});
+  return tile_aligned({fmt_is_w4(tf) ? g.a_pair : g.a, g.wp[0], g.wp[1], g.wp[2], g.ws[0], g.ws[1],
+                       g.ws[2], g.out[0], g.out[1], g.out[2]});
 }
 
 // Dense products (dense GEMM, fused QKV, MXFP4 GEMM) from 16 rows: the prefill
@@ -3418,8 +3414,8 @@ static int moe_forward_common(bool mx, const uint16_t* x, const float* logits, c
   const bool tile = mt == 4 && !f8 && tile_format(fmt, group) >= 0 && h % 128 == 0 && i % 128 == 0 &&
                     i * h <= kMaxDirectBytes &&
                     workspace_bytes >= static_cast<int64_t>(l.total) &&
-                    tile_aligned({workspace}, {mx ? x : nullptr, w1_packed, w3_packed, w2_packed,
-                                               w1_scales, w3_scales, w2_scales});
+                    tile_aligned({workspace, mx ? x : nullptr, w1_packed, w3_packed, w2_packed,
+                                  w1_scales, w3_scales, w2_scales});
   // W4A16 on 64-row tiles: x and the activations go in paired
   const bool paired = !mx && tile;
   // ...and when the batch takes the router launch (the 64-row tiles route

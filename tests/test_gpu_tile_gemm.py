@@ -212,8 +212,8 @@ def _shifted(t, by):
 @pytest.mark.parametrize("by", [4, 8, 12])
 @pytest.mark.parametrize("weights", ["g32", "g64", "g128", "mxfp4"])
 def test_operands_on_any_dword_keep_the_prefill_gemm(rng, weights, by):
-    """Codes, scales and rows on a dword that no 16-byte line starts at: the same
-    bits, from the same kernel (a dense W4A16 call writes its workspace)."""
+    """Codes, scales, rows and outputs on a dword that no 16-byte line starts at:
+    the same bits, from the same kernel (a dense W4A16 call writes its workspace)."""
     from local_kimi_amd import _lib
     from local_kimi_amd._lib import forced_path
     from local_kimi_amd.kernels import mxfp4_gemm, mxfp4_moe_block, w4a16_moe_forward
@@ -233,7 +233,8 @@ def test_operands_on_any_dword_keep_the_prefill_gemm(rng, weights, by):
         for args in ((dx, dp, ds), tuple(_shifted(t, by) for t in (dx, dp, ds))):
             ws = torch.full((_lib.query("lk_dense_gemm_workspace", m, n, k, group, 1, 0),), 0xA5,
                             dtype=torch.uint8, device=DEV)
-            y = torch.empty((m, n), dtype=torch.bfloat16, device=DEV)
+            y = torch.empty((m * n,), dtype=torch.bfloat16, device=DEV)
+            y = _shifted(y, 0 if args[0] is dx else by)
             _lib.call("lk_w4a16_dense_gemm_ws", *(t.data_ptr() for t in args), y.data_ptr(), m, n, k,
                       group, ws.data_ptr(), ws.numel(), stream)
             assert not bool((ws == 0xA5).all()), "not the prefill GEMM"

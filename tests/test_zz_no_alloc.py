@@ -150,7 +150,7 @@ def test_static_scratch_at_the_edge_of_its_size(banks, group):
 
 
 def test_workspace_off_its_alignment(banks):
-    """A workspace at 4 bytes off, which the direct loads do not take."""
+    """A workspace on a dword that no 16-byte line starts at."""
     run = _small_call(32, 8, 4, 420, 256, 256, 9)
     for a, b in zip(run(False), run(False, 4)):
         assert torch.equal(a, b)
