@@ -396,12 +396,11 @@ LK_API int lk_mxfp4_swiglu_gemm(const uint16_t* x, const int64_t* expert_indices
 
 /* The MoE block of lk_w4a16_moe_forward with MXFP4 expert banks (the
  * Kimi-Linear SwiGLU block; workspace from lk_mxfp4_moe_forward_workspace).
- * With h and i multiples of 128, prefill-sized calls (64-row expert tiles,
- * more than 2048 token-routes) run the expert GEMMs on the scaled fp4 MFMA
- * (v_mfma_scale_f32_16x16x128_f8f6f4): raw E2M1 weights and E8M0 exponents,
- * activations split into fp8 hi + lo (lk_mxfp4_split_activations); decode
- * sizes use bf16 MFMA on weights decoded by the scaled fp4 convert. The
- * environment variable LK_MXFP4_MFMA=fp4 or =bf16 forces one form. */
+ * The expert GEMMs run on bf16 MFMA, on weights decoded by the scaled fp4
+ * convert. The path knob mxfp4_mfma=fp4 takes the scaled fp4 MFMA
+ * (v_mfma_scale_f32_16x16x128_f8f6f4) where h and i are multiples of 128: raw
+ * E2M1 weights and E8M0 exponents, activations split into fp8 hi + lo
+ * (lk_mxfp4_split_activations). */
 LK_API int64_t lk_mxfp4_moe_forward_workspace(int64_t tokens, int64_t experts, int64_t h,
                                               int64_t i, int64_t top_k);
 LK_API int lk_mxfp4_moe_forward(const uint16_t* x, const float* logits, const float* bias,

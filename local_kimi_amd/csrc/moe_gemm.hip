@@ -2856,8 +2856,8 @@ constexpr int64_t kStreamSmallEntries = 2048;
 // scaled fp4 MFMA (raw fp4 weights, activations split into fp8 hi + lo). The
 // split keeps bf16 precision but takes two scaled MFMAs per 128-wide k-step,
 // the same MFMA time as four bf16 ones, plus two split launches: a 2048-token
-// Kimi-Linear layer measured 581 us in the bf16 form against 620 us, and 64
-// tokens 145 against 196 us.
+// Kimi-Linear layer measured 395 us in the bf16 form (the prefill GEMM) against
+// 622 us, and 64 tokens 133 against 196 us.
 bool mxfp4_scaled_mfma() { return path_choice(kKnobMxfp4Mfma) == 1; }
 
 // 16-row tiles -> 1, 64-row tiles -> 4, the LDS-staged kernel -> 0.
